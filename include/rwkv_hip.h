@@ -319,14 +319,13 @@ rwkv_status rwkv_sym_gemv_ep(const float* x, int64_t N,
  * relu(·)² as fp16 (y is then an fp16 buffer; cmix's key, exact in fp16).
  * workspace: NULL, or device memory of rwkv_quant_gemm_workspace(M, OUT, IN)
  * bytes (16-byte aligned; a smaller one is refused before any launch).  With
- * it, shapes with few 128 × 128 output tiles split the K sum into ranges
- * summed in a fixed order by a second kernel (the same bound, deterministic,
- * far faster for a few hundred rows), and shapes with at least 128 output
- * tiles of 256 × 256 and f16 inputs dequantise the weight into the
- * workspace (rwkv_sb6_dequant / rwkv_sym_dequant, f16) and run rwkv_f16_gemm
- * over it — the same products in the same order, so bitwise the one-range
- * result, at 2-2.5x its speed for M >= 4096.  With NULL the launch is one
- * range.  Launches sharing a workspace must not overlap. */
+ * it, passes of few output tiles split the K sum over the waves of a workgroup
+ * (a fixed order: deterministic, the same bound), and larger ones dequantise
+ * the weight into the workspace (fp16, the dequant's values in the matrix
+ * cores' order) and multiply from there — the same products in the same order
+ * as one range, so bitwise its result.  Which one depends on the shape alone:
+ * f32 inputs give the bits of f16 inputs of equal values.  With NULL the launch
+ * is one range.  Launches sharing a workspace must not overlap. */
 int rwkv_sb6_gemm_applies(int64_t OUT, int64_t IN, int xbits, int64_t out_per);
 int64_t rwkv_quant_gemm_workspace(int64_t M, int64_t OUT, int64_t IN);
 rwkv_status rwkv_sb6_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda, int64_t x_group_stride,

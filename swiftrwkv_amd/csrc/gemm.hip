@@ -6,16 +6,16 @@
 // (X070Backbone.baseMatmul, Sources/RWKVGen/X070Backbone.swift:337-356,
 // 733-739; the dequant of RwkvqDequant.swift:116-140 (sb6) and :350-388,
 // 442-466 (sym, whose fp16 branch computes in half)).  Here the dequant
-// happens in the GEMM's operand path (quant_gemm_kernel: no dense weight is
-// written), or, for shapes with many output tiles, once per matrix into a
-// workspace that dense_gemm_kernel then multiplies (below).  Per
+// happens in the GEMM's operand path (quant_gemm_kernel; gemm_ks_kernel for
+// passes of few output tiles), or, for larger ones, once per matrix into a
+// workspace that dense_tiles_kernel then multiplies (gemm_route).  Per
 // element the numbers are the reference's: the weight is exactly what the
 // dequant kernels store in fp16 — sb6 fp16(fma(code, half(qs·d), half(qm·dm))),
 // sym fp16((code − bias)·half(qs·d)) — the input is rounded to fp16, products
 // accumulate in fp32 on v_mfma_f32_16x16x32_f16, and the sum is rounded to
 // fp16 (the fp16 matmul's output) before the epilogue.
 //
-// Tiling.  A workgroup of 4 waves computes a 128 (input rows) × 128 (output
+// quant_gemm_kernel.  A workgroup of 4 waves computes a 128 (input rows) × 128 (output
 // features) tile in stages of 64 columns (two 32-column units); two
 // workgroups share a CU.  The input tile is staged in LDS as fp16
 // (double-buffered; rows padded to 144 B so the 16 lanes of a row group read
@@ -35,6 +35,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "launch.h"
 
@@ -42,8 +43,10 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BK = 64;            // columns per stage: two sb6 units
+constexpr int DKS = 64;           // columns per stage of the dense kernels
 constexpr int LDS_ROW = BK + 8;   // halves per staged row (144 B)
 
 __device__ __forceinline__ float f16f(uint32_t bits16) {
@@ -60,8 +63,6 @@ struct GemmArgs {
     void* y;              // [M][ldy]: fp32 (epilogues 0, 1) or fp16 (epilogue 2)
     int64_t ldy;
     int M, N, K, out_per;
-    float* part;          // splits > 1: the fp32 partial sums [splits][M][N]
-    int splits;           // K ranges the tile's stages are divided into
 };
 
 // The epilogue of one output: fp16 rounding of the fp32 sum (the fp16
@@ -77,6 +78,26 @@ __device__ __forceinline__ void store_out(void* y, int64_t idx, float acc) {
     } else {
         const float rl = fmaxf(v, 0.0f);
         reinterpret_cast<_Float16*>(y)[idx] = (_Float16)(rl * rl);
+    }
+}
+
+// store_out of four consecutive outputs, 4-element aligned.
+template <int EP>
+__device__ __forceinline__ void store_out4(void* y, int64_t idx, f32x4 acc) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = hround(acc[c]);
+    if constexpr (EP == 2) {
+        typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+        half4 h;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float rl = fmaxf(acc[c], 0.0f);
+            h[c] = (_Float16)(rl * rl);
+        }
+        *reinterpret_cast<half4*>(reinterpret_cast<_Float16*>(y) + idx) = h;
+    } else {
+        f32x4* p = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(y) + idx);
+        *p = EP == 1 ? *p + acc : acc;
     }
 }
 
@@ -116,37 +137,56 @@ __device__ __forceinline__ half8 bytes8_fma(uint32_t c0, uint32_t c1, float s, f
 template <int XB>
 struct Sb6W {
     static constexpr int UB = 16 + 4 * XB;
-    struct Raw {
+    static constexpr int SPS = 2;   // s2 halves per super-block
+    struct Codes {
         uint2 nib[2];
         uint32_t hi[2][XB > 0 ? XB : 1];
+    };
+    struct Raw {
+        Codes c;
         uint32_t sm;   // qsqm of units u, u + 1
         uint32_t dd;   // ddm of their super-block
     };
-    __device__ static Raw load(const GemmArgs& g, int64_t row, int u, int gq) {
-        const int NU = g.K >> 5, NSB = g.K >> 8;
-        Raw r;
+    // a row's codes of units u, u + 1, at unit u's bytes
+    __device__ static Codes load_codes(const uint8_t* pq, int gq) {
+        Codes r;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            const uint8_t* b = g.q + (row * NU + u + q) * UB;
+            const uint8_t* b = pq + q * UB;
             // 4-byte aligned only for a 20-byte unit: two dword loads
             const uint32_t* w = reinterpret_cast<const uint32_t*>(b + 8 * (gq & 1));
             r.nib[q] = make_uint2(w[0], w[1]);
 #pragma unroll
             for (int e = 0; e < XB; ++e) r.hi[q][e] = *reinterpret_cast<const uint32_t*>(b + 16 + 4 * e);
         }
+        return r;
+    }
+    __device__ static Raw load(const GemmArgs& g, int64_t row, int u, int gq) {
+        const int NU = g.K >> 5, NSB = g.K >> 8;
+        Raw r;
+        r.c = load_codes(g.q + (row * NU + u) * UB, gq);
         r.sm = *reinterpret_cast<const uint32_t*>(g.s1 + (row * NU + u) * 2);
         r.dd = *reinterpret_cast<const uint32_t*>(g.s2 + (row * NSB + (u >> 3)) * 2);
         return r;
     }
-    __device__ static half8 dequant(const Raw& r, int q, int gq) {
-        const uint32_t sm = r.sm >> (16 * q);
+    // a unit's scale word for decode(): (half(qs·d), half(qm·dm)) from its qsqm and its super-block's ddm
+    __device__ static uint32_t scale(uint32_t sm, uint32_t dd) {
+        const _Float16 s = (_Float16)((float)(sm & 0xffu) * f16f(dd));
+        const _Float16 m = (_Float16)((float)(int8_t)((sm >> 8) & 0xffu) * f16f(dd >> 16));
+        return (uint32_t)__builtin_bit_cast(uint16_t, s) | ((uint32_t)__builtin_bit_cast(uint16_t, m) << 16);
+    }
+    __device__ static uint32_t load_scale(const GemmArgs& g, int64_t row, int u) {
+        const int NU = g.K >> 5, NSB = g.K >> 8;
+        return scale(*reinterpret_cast<const uint16_t*>(g.s1 + (row * NU + u) * 2),
+                     *reinterpret_cast<const uint32_t*>(g.s2 + (row * NSB + (u >> 3)) * 2));
+    }
+    __device__ static half8 decode(const Codes& r, int q, int gq, float s, float m) {
         const int shift = (gq >> 1) * 4;   // columns 16..31 in the high nibbles
         const uint32_t c0 = (r.nib[q].x >> shift) & 0x0F0F0F0Fu, c1 = (r.nib[q].y >> shift) & 0x0F0F0F0Fu;
-        const float m = hround((float)(int8_t)((sm >> 8) & 0xffu) * f16f(r.dd >> 16));
         if constexpr (XB == 0) {
             // a 4-bit code byte read as fp8 E4M3 is code·2^-9 exactly: two
             // codes widen per instruction and s carries the 2^9
-            const float s = hround((float)(sm & 0xffu) * f16f(r.dd)) * 512.0f;
+            s *= 512.0f;
             const auto p0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)c0, false);
             const auto p1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)c0, true);
             const auto p2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)c1, false);
@@ -162,7 +202,6 @@ struct Sb6W {
             h[7] = (_Float16)fmaf(p3[1], s, m);
             return h;
         } else {
-            const float s = hround((float)(sm & 0xffu) * f16f(r.dd));
             uint32_t a = c0, b = c1;
 #pragma unroll
             for (int e = 0; e < XB; ++e) {
@@ -172,6 +211,13 @@ struct Sb6W {
             }
             return bytes8_fma(a, b, s, m);
         }
+    }
+    // decode with a scale word of scale()
+    __device__ static half8 decode_scaled(const Codes& r, int q, int gq, uint32_t sw) {
+        return decode(r, q, gq, f16f(sw), f16f(sw >> 16));
+    }
+    __device__ static half8 dequant(const Raw& r, int q, int gq) {
+        return decode_scaled(r.c, q, gq, scale(r.sm >> (16 * q), r.dd));
     }
 };
 
@@ -184,18 +230,21 @@ struct Sb6W {
 template <int BITS>
 struct SymW {
     static constexpr int UB = BITS == 8 ? 32 : 24;
-    struct Raw {
+    static constexpr int SPS = 1;
+    struct Codes {
         uint2 c[2];
         uint32_t hi[2][BITS == 8 ? 1 : 2];
+    };
+    struct Raw {
+        Codes c;
         uint32_t qs;   // the four 16-column scales of units u, u + 1
         uint32_t d;    // super-block scale (fp16)
     };
-    __device__ static Raw load(const GemmArgs& g, int64_t row, int u, int gq) {
-        const int NU = g.K >> 5, NSB = g.K >> 8;
-        Raw r;
+    __device__ static Codes load_codes(const uint8_t* pq, int gq) {
+        Codes r;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            const uint8_t* b = g.q + (row * NU + u + q) * UB;
+            const uint8_t* b = pq + q * UB;
             if constexpr (BITS == 8) {
                 r.c[q] = *reinterpret_cast<const uint2*>(b + 8 * gq);
             } else {
@@ -204,12 +253,27 @@ struct SymW {
                 r.hi[q][1] = *reinterpret_cast<const uint32_t*>(b + 20);
             }
         }
-        r.qs = *reinterpret_cast<const uint32_t*>(g.s1 + row * (g.K >> 4) + 2 * u);
+        return r;
+    }
+    __device__ static Raw load(const GemmArgs& g, int64_t row, int u, int gq) {
+        const int NU = g.K >> 5, NSB = g.K >> 8;
+        Raw r;
+        r.c = load_codes(g.q + (row * NU + u) * UB, gq);
+        r.qs = *reinterpret_cast<const uint32_t*>(g.s1 + (row * NU + u) * 2);
         r.d = g.s2[row * NSB + (u >> 3)];
         return r;
     }
-    __device__ static half8 dequant(const Raw& r, int q, int gq) {
-        const float s = hround((float)(int8_t)((r.qs >> (8 * (2 * q + (gq >> 1)))) & 0xffu) * f16f(r.d));
+    // a unit's scale word: half(qs·d) of its columns 0..15 and 16..31
+    __device__ static uint32_t scale(uint32_t qs, uint32_t d) {
+        const _Float16 a = (_Float16)((float)(int8_t)(qs & 0xffu) * f16f(d));
+        const _Float16 b = (_Float16)((float)(int8_t)((qs >> 8) & 0xffu) * f16f(d));
+        return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+    }
+    __device__ static uint32_t load_scale(const GemmArgs& g, int64_t row, int u) {
+        const int NU = g.K >> 5, NSB = g.K >> 8;
+        return scale(*reinterpret_cast<const uint16_t*>(g.s1 + (row * NU + u) * 2), g.s2[row * NSB + (u >> 3)]);
+    }
+    __device__ static half8 decode(const Codes& r, int q, int gq, float s) {
         if constexpr (BITS == 8) {
             // int8 codes as unsigned bytes code + 128: (u − 128)·s exactly
             return bytes8_fma(r.c[q].x ^ 0x80808080u, r.c[q].y ^ 0x80808080u, s, -128.0f * s);
@@ -224,6 +288,12 @@ struct SymW {
             }
             return bytes8_fma(a, b, s, -32.0f * s);
         }
+    }
+    __device__ static half8 decode_scaled(const Codes& r, int q, int gq, uint32_t sw) {
+        return decode(r, q, gq, f16f(sw >> (16 * (gq >> 1))));
+    }
+    __device__ static half8 dequant(const Raw& r, int q, int gq) {
+        return decode(r.c, q, gq, hround((float)(int8_t)((r.qs >> (8 * (2 * q + (gq >> 1)))) & 0xffu) * f16f(r.d)));
     }
 };
 
@@ -243,15 +313,14 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
     // every feature tile of one block before the next, so an input block is
     // fetched into one L2 only.  The grid is padded to whole groups of 8 row
     // blocks; a padding workgroup exits before any barrier.
-    const int ntn = g.N / BN, S = g.splits;
-    const int total = ((g.M + BM - 1) / BM) * ntn * S;
+    const int ntn = g.N / BN;
+    const int total = ((g.M + BM - 1) / BM) * ntn;
     const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
-    const int t = xcd * (total >> 3) + min(xcd, total & 7) + loc;   // the tile's place in (m, n, split) order
-    const int kz = t % S, tile_n = (t / S) % ntn, tile_m = t / (S * ntn);
+    const int t = xcd * (total >> 3) + min(xcd, total & 7) + loc;   // the tile's place in (m, n) order
+    const int tile_n = t % ntn, tile_m = t / ntn;
     const int n0 = tile_n * BN;
     const int m0 = tile_m * BM;
     const int nst = g.K / BK;
-    const int st0 = (int)((int64_t)kz * nst / S), st1 = (int)((int64_t)(kz + 1) * nst / S);
 
     // input rows of this tile come from the matrix group its output features belong to
     const TA* xg = reinterpret_cast<const TA*>(g.x) + (int64_t)(n0 / g.out_per) * g.x_gstride;
@@ -318,8 +387,8 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
         }
     };
 
-    auto ar = load_a(st0);
-    BRaw bcur = load_b(st0);
+    auto ar = load_a(0);
+    BRaw bcur = load_b(0);
     store_a(0, ar);
     half8 b0[NT], b1[NT];
     dequant(bcur, 0, b0);
@@ -328,9 +397,9 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
     // Per stage: the next stage's bytes are requested first; unit 0's
     // products run while unit 1 is decoded, unit 1's while the next stage's
     // unit 0 is (one MFMA, one VALU instruction, alternately).
-    for (int st = st0; st < st1; ++st) {
-        const int buf = (st - st0) & 1;
-        const bool more = st + 1 < st1;
+    for (int st = 0; st < nst; ++st) {
+        const int buf = st & 1;
+        const bool more = st + 1 < nst;
         BRaw bnxt = bcur;
         if (more) {
             ar = load_a(st + 1);
@@ -355,19 +424,6 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
         __syncthreads();
     }
 
-    if (S > 1) {   // this K range's fp32 sums; gemm_split_reduce adds the ranges and applies the epilogue
-        float* part = g.part + (int64_t)kz * g.M * g.N;
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = m0 + 16 * i + 4 * gq + r;
-                if (row >= g.M) continue;
-#pragma unroll
-                for (int j = 0; j < NT; ++j) part[(int64_t)row * g.N + nb + 16 * j] = acc[i][j][r];
-            }
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
 #pragma unroll
@@ -380,13 +436,443 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
     }
 }
 
-// ── dense fp16 weights ──
+// ── few output tiles: the K sum split over the waves of a workgroup ──
+//
+// A pass of a few hundred rows has few output tiles, and a tile whose K stages
+// run one after another waits on memory once per stage.  Here a workgroup is
+// one tile of 16·MT × 16·NT outputs and its W waves take K / W columns each.
+// A wave works alone: it moves 128 columns at a time (its input rows and its
+// weight rows' packed bytes) through its own LDS region, so no barrier stands
+// in the K loop, with the next 128 columns' loads in registers meanwhile; the
+// W partial tiles meet in LDS at the end, summed in wave order
+// (deterministic), where the epilogue is applied.  One launch.
+//
+// Why through LDS: an MFMA operand wants lane l to hold row l & 15, and a load
+// in that shape has every lane in another cache line (measured ~50 cycles per
+// load instruction and CU, against 16 for one whose lanes run along a row:
+// 128 rows × 768 × 3072 took 11.8 µs that way, 7.0 like this, on 32 × 16 tiles).
+// Past a tile's start its time is its bytes through the CU's one memory path
+// (18 KB per 64 × 32 × 128 step) beside as long a stretch of decoding.
+// The scale words of the wave's rows go through its region too, four steps at
+// a time (read per step they would cost as many cache lines as the codes).
+constexpr int KS_COLS = 2 * BK;            // columns per step: four units
+constexpr int KS_PAD = 4;                  // partial tiles: row padding (floats)
+constexpr size_t KS_LDS = 160 * 1024;      // a gfx950 workgroup's LDS
+constexpr int KS_AROW = KS_COLS * 2 + 16;  // LDS bytes per staged input row: an odd number of 16-byte chunks
+// steps per block of scale words, and LDS bytes per weight row of them (an odd number of chunks)
+constexpr int ks_ssteps(int nt) { return nt == 4 ? 2 : 4; }
+constexpr int ks_srow(int nt) { return ks_ssteps(nt) * 16 + 16; }
+
+struct KsArgs {
+    GemmArgs g;
+    int ep;    // epilogue (store_out)
+    int vec;   // y rows take aligned 4-wide stores
+};
+
+// LDS bytes per staged weight row: the four units' bytes in an odd number of
+// 16-byte chunks, so 16 rows' reads at one column fall on distinct banks.
+template <class F>
+constexpr int ks_brow() {
+    constexpr int chunks = 4 * F::UB / 16;
+    return 16 * (chunks | 1);
+}
+template <class F>
+constexpr int ks_wave_lds(int mt, int nt) {
+    return 16 * mt * KS_AROW + 16 * nt * (ks_brow<F>() + ks_srow(nt));
+}
+
+template <class F, typename TA, int MT, int NT, int MAXW>
+__global__ __launch_bounds__(64 * MAXW) void gemm_ks_kernel(KsArgs ka) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // W wave regions, then the partial tiles
+    const GemmArgs& g = ka.g;
+    constexpr int BM = 16 * MT, BN = 16 * NT, LS = BN + KS_PAD, SS = ks_ssteps(NT), SR = ks_srow(NT);
+    constexpr int AC = KS_COLS * (int)sizeof(TA) / 16;   // 16-byte chunks per input row and step
+    constexpr int AL = BM * AC / 64;                     // input loads per lane
+    constexpr int BC = 4 * F::UB / 16;                   // chunks per weight row and step
+    constexpr int BL = (BN * BC + 63) / 64;              // weight loads per lane
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int W = blockDim.x >> 6;
+    const int gq = lane >> 4, li = lane & 15;
+    // an XCD takes a contiguous run of tiles, row blocks fastest: the row
+    // blocks of a weight panel share one L2
+    const int tm = (g.M + BM - 1) / BM, total = tm * (g.N / BN);
+    const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
+    const int t = xcd * (total >> 3) + min(xcd, total & 7) + loc;
+    const int m0 = (t % tm) * BM, n0 = (t / tm) * BN;
+    const int steps = g.K / KS_COLS, NU = g.K >> 5;
+    const int p0 = wave * steps / W, p1 = (wave + 1) * steps / W;   // W <= steps: at least one step each
+
+    unsigned char* const mine = lds + wave * ks_wave_lds<F>(MT, NT);
+    unsigned char* const mb = mine + BM * KS_AROW;
+    unsigned char* const ms = mb + BN * ks_brow<F>();
+
+    // Uniform bases (tile, step) plus a 32-bit offset per load.
+    const char* xt = reinterpret_cast<const char*>(reinterpret_cast<const TA*>(g.x) +
+                                                   (int64_t)(n0 / g.out_per) * g.x_gstride + (int64_t)m0 * g.lda);
+    const uint8_t* qt = g.q + (int64_t)n0 * NU * F::UB;
+    uint32_t xo[AL], bo[BL];
+#pragma unroll
+    for (int e = 0; e < AL; ++e) {
+        const int id = lane + 64 * e, row = id / AC, c = id % AC;
+        xo[e] = (uint32_t)(min(row, g.M - 1 - m0) * (int)g.lda * (int)sizeof(TA) + 16 * c);
+    }
+#pragma unroll
+    for (int e = 0; e < BL; ++e) {
+        const int id = min(lane + 64 * e, BN * BC - 1), row = id / BC, c = id % BC;
+        bo[e] = (uint32_t)(row * NU * F::UB + 16 * c);
+    }
+    u32x4 ra[AL], rb[BL];
+    auto load = [&](int p) __attribute__((always_inline)) {
+        const char* xs = xt + (int64_t)p * (KS_COLS * (int)sizeof(TA));
+        const uint8_t* qs = qt + (int64_t)p * (4 * F::UB);
+#pragma unroll
+        for (int e = 0; e < BL; ++e) rb[e] = *reinterpret_cast<const u32x4*>(qs + bo[e]);
+#pragma unroll
+        for (int e = 0; e < AL; ++e) ra[e] = *reinterpret_cast<const u32x4*>(xs + xo[e]);
+    };
+    auto stage = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < BL; ++e) {
+            const int id = min(lane + 64 * e, BN * BC - 1);
+            *reinterpret_cast<u32x4*>(mb + id / BC * ks_brow<F>() + id % BC * 16) = rb[e];
+        }
+#pragma unroll
+        for (int e = 0; e < AL; ++e) {
+            const int id = lane + 64 * e, row = id / AC, c = id % AC;
+            unsigned char* const r = mine + row * KS_AROW;
+            if constexpr (sizeof(TA) == 2) {
+                *reinterpret_cast<u32x4*>(r + 16 * c) = ra[e];
+            } else {
+                typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+                half4 h;
+                h[0] = (_Float16)__uint_as_float(ra[e].x); h[1] = (_Float16)__uint_as_float(ra[e].y);
+                h[2] = (_Float16)__uint_as_float(ra[e].z); h[3] = (_Float16)__uint_as_float(ra[e].w);
+                *reinterpret_cast<half4*>(r + 8 * c) = h;
+            }
+        }
+    };
+    // Scale words of steps p .. p + 3 of the wave's rows: lane → (row, step),
+    // its four units' bytes and their super-block's fp16 scales.
+    constexpr int SL = BN * SS / 64;
+    const int NSB = g.K >> 8;
+    uint2 rs[SL];
+    uint32_t rd[SL];
+    auto load_scales = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < SL; ++e) {
+            const int id = lane + 64 * e, row = n0 + id / SS, st = min(p + id % SS, steps - 1);
+            rs[e] = *reinterpret_cast<const uint2*>(g.s1 + ((int64_t)row * NU + 4 * st) * 2);
+            const uint16_t* d = g.s2 + ((int64_t)row * NSB + (st >> 1)) * F::SPS;
+            if constexpr (F::SPS == 2) rd[e] = *reinterpret_cast<const uint32_t*>(d);
+            else rd[e] = *d;
+        }
+    };
+    auto stage_scales = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < SL; ++e) {
+            const int id = lane + 64 * e;
+            u32x4 w;
+            w[0] = F::scale(rs[e].x, rd[e]);
+            w[1] = F::scale(rs[e].x >> 16, rd[e]);
+            w[2] = F::scale(rs[e].y, rd[e]);
+            w[3] = F::scale(rs[e].y >> 16, rd[e]);
+            *reinterpret_cast<u32x4*>(ms + id / SS * SR + id % SS * 16) = w;
+        }
+    };
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto products = [&](int p) __attribute__((always_inline)) {
+        u32x4 sw[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            sw[j] = *reinterpret_cast<const u32x4*>(ms + (16 * j + li) * SR + (p - p0) % SS * 16);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            typename F::Codes cd[NT];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) cd[j] = F::load_codes(mb + (16 * j + li) * ks_brow<F>() + 2 * h * F::UB, gq);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                half8 b[NT];
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const uint32_t s = h == 0 ? (q == 0 ? sw[j].x : sw[j].y) : (q == 0 ? sw[j].z : sw[j].w);
+                    b[j] = F::decode_scaled(cd[j], q, gq, s);
+                }
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    const half8 a = *reinterpret_cast<const half8*>(mine + (16 * i + li) * KS_AROW +
+                                                                    (4 * (2 * h + q) + gq) * 16);
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[j], acc[i][j], 0, 0, 0);
+                }
+            }
+        }
+    };
+    load_scales(p0);
+    load(p0);
+    auto next_scales = [&](int p) __attribute__((always_inline)) {
+        if ((p - p0) % SS != 0) return;
+        stage_scales();
+        load_scales(p + SS);
+    };
+    // the last step is peeled, so no input or code load is repeated
+    for (int p = p0; p < p1 - 1; ++p) {
+        next_scales(p);
+        stage();
+        load(p + 1);
+        products(p);
+    }
+    next_scales(p1 - 1);
+    stage();
+    products(p1 - 1);
+    __syncthreads();   // the staging LDS becomes the partial tiles
+
+    float* const part = reinterpret_cast<float*>(lds);   // [W][BM][LS]
+    float* const own = part + wave * (BM * LS);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) own[(16 * i + 4 * gq + r) * LS + 16 * j + li] = acc[i][j][r];
+    __syncthreads();
+    for (int q = threadIdx.x; q < BM * BN / 4; q += blockDim.x) {
+        const int row = q / (BN / 4), col = q % (BN / 4) * 4;
+        const float* src = part + row * LS + col;
+        f32x4 v = *reinterpret_cast<const f32x4*>(src);
+        for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(src + k * (BM * LS));
+        if (m0 + row >= g.M) continue;
+        const int64_t at = (int64_t)(m0 + row) * g.ldy + n0 + col;
+        if (!ka.vec) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if (ka.ep == 0) store_out<0>(g.y, at + c, v[c]);
+                else if (ka.ep == 1) store_out<1>(g.y, at + c, v[c]);
+                else store_out<2>(g.y, at + c, v[c]);
+            }
+            continue;
+        }
+        if (ka.ep == 0) store_out4<0>(g.y, at, v);
+        else if (ka.ep == 1) store_out4<1>(g.y, at, v);
+        else store_out4<2>(g.y, at, v);
+    }
+}
+
+// ── dequantised weights in operand order ──
+//
+// For a quantised matrix the workspace copy need not be row-major: it is
+// written in the order the matrix cores read it, so the GEMM loads its weight
+// operands straight into registers and only the inputs go through LDS.  Block
+// (n16, u) of 16 rows × one 32-column unit is 1 KiB at index n16·(K/32) + u;
+// lane gq·16 + li's 16 bytes are row 16·n16 + li, columns 32u + 8gq .. + 7.
+// (The row-major kernel below is bound by LDS: per 64-column stage its eight
+// waves read 192 KB and write 64 KB, ~2,560 cycles at 128 and 64 B per cycle
+// against 2,048 of MFMA.)
+template <class F>
+__global__ __launch_bounds__(256) void dequant_tiles_kernel(GemmArgs g, _Float16* __restrict__ out) {
+    const int NU = g.K >> 5, NSB = g.K >> 8;
+    const int lane = threadIdx.x & 63, gq = lane >> 4, li = lane & 15;
+    // one wave: 16 rows × half a super-block (four units)
+    const int wv = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (wv >= (g.N >> 4) * 2 * NSB) return;
+    const int n16 = wv / (2 * NSB), hb = wv - n16 * 2 * NSB, u0 = 4 * hb;
+    const int64_t row = 16 * n16 + li;
+    const uint2 sm = *reinterpret_cast<const uint2*>(g.s1 + (row * NU + u0) * 2);
+    uint32_t dd;
+    if constexpr (F::SPS == 2) dd = *reinterpret_cast<const uint32_t*>(g.s2 + (row * NSB + (hb >> 1)) * 2);
+    else dd = g.s2[row * NSB + (hb >> 1)];
+    const uint8_t* pq = g.q + (row * NU + u0) * F::UB;
+    const typename F::Codes c[2] = {F::load_codes(pq, gq), F::load_codes(pq + 2 * F::UB, gq)};
+    half8* o = reinterpret_cast<half8*>(out) + ((int64_t)n16 * NU + u0) * 64 + lane;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        o[64 * u] = F::decode_scaled(c[u >> 1], u & 1, gq, F::scale((u < 2 ? sm.x : sm.y) >> (16 * (u & 1)), dd));
+}
+
+// The dense product over a weight in operand order.  Tile 16·WM·AM input rows
+// × 16·WN·AN features, WM × WN waves, 64-column stages (two units).  Inputs:
+// global → registers a stage ahead → LDS (rows of 128 B, chunk c of row r at
+// c ^ (r & 7)), two buffers.  Weights: two stages of operands in registers,
+// a unit's set reloaded as soon as its products are issued.  The weight is the
+// MFMA's A operand and the input its B operand, so lane gq·16 + li ends with
+// input row li, features 4gq .. 4gq + 3: four consecutive outputs to store.
+// Per output the products and their order are quant_gemm_kernel's.
+struct DenseTArgs {
+    const void* x;       // [groups][M][lda], fp16 or fp32
+    int64_t lda, x_gstride;
+    const _Float16* w;   // operand order
+    void* y;             // [M][ldy]
+    int64_t ldy;
+    int M, N, K, out_per;
+    int vec;             // y rows take aligned 4-wide accesses
+};
+
+template <typename TA, int EP, int WM, int WN, int AM, int AN, int DP, int DA>
+__global__ __launch_bounds__(64 * WM * WN, WM * WN > 4 ? 1 : 2) void dense_tiles_kernel(DenseTArgs g) {
+    constexpr int XV = (int)sizeof(TA) / 2;   // 16-byte loads per chunk of 8 inputs
+    constexpr int TM = 16 * WM * AM, TN = 16 * WN * AN;
+    constexpr int RP = 8 * WM * WN;   // rows one pass of the workgroup's input loads covers
+    constexpr int PX = TM / RP;       // input chunks per thread and stage
+    __shared__ u32x4 lds[2][TM * 8];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int gq = lane >> 4, li = lane & 15;
+    // Tiles in groups of 4 row blocks × every feature block, feature-major
+    // within a group; XCD x (workgroups x, x + 8, ...) takes a contiguous run
+    // of that order.
+    const int ntm = (g.M + TM - 1) / TM, ntn = g.N / TN, total = ntm * ntn;
+    const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
+    const int t = xcd * (total >> 3) + min(xcd, total & 7) + loc;
+    const int grp = t / (4 * ntn), first = 4 * grp, gm = min(4, ntm - first);
+    const int rr = t - grp * 4 * ntn;
+    const int m0 = (first + rr % gm) * TM, n0 = (rr / gm) * TN;
+    const int NU = g.K >> 5, nst = g.K / DKS;
+
+    const int c = tid & 7, r0 = tid >> 3;
+    const int mrows = min(TM, g.M - m0);
+    const TA* xt = reinterpret_cast<const TA*>(g.x) + (int64_t)(n0 / g.out_per) * g.x_gstride + (int64_t)m0 * g.lda;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<TA*>(xt), 0, (int)(mrows * g.lda * (int)sizeof(TA)), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<_Float16*>(g.w + (int64_t)n0 * g.K), 0, (int)((int64_t)TN * g.K * 2), 0x00020000);
+    uint32_t xo[PX];
+#pragma unroll
+    for (int p = 0; p < PX; ++p) xo[p] = (uint32_t)((min(r0 + RP * p, mrows - 1) * (int)g.lda + 8 * c) * (int)sizeof(TA));
+    const int dst0 = r0 * 8 + (c ^ (r0 & 7));   // row r0 + RP·p: + 8·RP·p chunks, the same swizzle
+    const int wm = wave % WM, wn = wave / WM;
+    u32x4 v[DA][PX * XV];
+    auto gload = [&](u32x4 (&d)[PX * XV], int st) __attribute__((always_inline)) {
+        const uint32_t so = (uint32_t)(min(st, nst - 1) * DKS * (int)sizeof(TA));
+#pragma unroll
+        for (int p = 0; p < PX; ++p)
+#pragma unroll
+            for (int e = 0; e < XV; ++e)
+                d[p * XV + e] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xo[p] + 16 * e, so, 0));
+    };
+    auto swrite = [&](int buf, const u32x4 (&d)[PX * XV]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < PX; ++p) {
+            if constexpr (XV == 1) {
+                lds[buf][dst0 + 8 * RP * p] = d[p];
+            } else {
+                half8 h;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    h[e] = (_Float16)__uint_as_float(d[2 * p][e]);
+                    h[4 + e] = (_Float16)__uint_as_float(d[2 * p + 1][e]);
+                }
+                lds[buf][dst0 + 8 * RP * p] = __builtin_bit_cast(u32x4, h);
+            }
+        }
+    };
+    half8 bq[DP][2][AN];   // [stage mod DP][unit][feature tile]
+    const uint32_t wlane = (uint32_t)(lane * 16);
+    auto wload = [&](half8 (&b)[AN], int st, int kk) __attribute__((always_inline)) {
+        const int u = 2 * min(st, nst - 1) + kk;
+#pragma unroll
+        for (int j = 0; j < AN; ++j)
+            b[j] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 rw, wlane, (uint32_t)(((wn * AN + j) * NU + u) * 1024), 0));
+    };
+    f32x4 acc[AM][AN];
+#pragma unroll
+    for (int a = 0; a < AM; ++a)
+#pragma unroll
+        for (int b = 0; b < AN; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int ra = (16 * AM * wm + li) * 8;
+    auto operands = [&](int buf, int kk, half8 (&av)[AM]) __attribute__((always_inline)) {
+        const int ch = (4 * kk + gq) ^ (li & 7);
+#pragma unroll
+        for (int a = 0; a < AM; ++a) av[a] = __builtin_bit_cast(half8, lds[buf][ra + 128 * a + ch]);
+    };
+    auto products = [&](const half8 (&av)[AM], const half8 (&bv)[AN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int a = 0; a < AM; ++a)
+#pragma unroll
+            for (int b = 0; b < AN; ++b)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[b], av[a], acc[a][b], 0, 0, 0);
+    };
+    // Stage st, at place q of the unrolled DP (LDS buffer q & 1).  Unit 0's
+    // products carry the reload of the unit-1 operands the previous stage
+    // consumed, unit 1's the reload of unit 0's, the LDS write of the next
+    // stage's inputs and the loads that refill their registers.
+    auto stage = [&](int q, int st) __attribute__((always_inline)) {
+        {
+            half8 av[AM];
+            operands(q & 1, 0, av);
+            wload(bq[(q + DP - 1) % DP][1], st + DP - 1, 1);
+            products(av, bq[q][0]);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // DS reads
+#pragma unroll
+            for (int i = 0; i < AM; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, AN, 0);   // MFMA
+                if (i < AM - 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, (AN + AM - 1) / AM, 0);   // VMEM read
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        {
+            half8 av[AM];
+            operands(q & 1, 1, av);
+            wload(bq[q][0], st + DP, 0);
+            products(av, bq[q][1]);
+            swrite((q & 1) ^ 1, v[(q + 1) % DA]);
+            gload(v[(q + 1) % DA], st + 1 + DA);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+            for (int i = 0; i < AM; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, AN, 0);
+                if (i < AM - 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x200, (PX + AM - 1) / AM, 0);        // DS write
+                __builtin_amdgcn_sched_group_barrier(0x020, (AN + PX * XV + AM - 1) / AM, 0);   // VMEM read
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
+
+    // nst is a multiple of DP; loads past the last stage repeat it, and the
+    // final LDS write lands in a buffer no later stage reads
+    gload(v[0], 0);
+#pragma unroll
+    for (int d = 0; d < DP; ++d) {
+        wload(bq[d][0], d, 0);
+        if (d < DP - 1) wload(bq[d][1], d, 1);
+    }
+    swrite(0, v[0]);
+#pragma unroll
+    for (int d = 1; d <= DA; ++d) gload(v[d % DA], d);
+    __syncthreads();
+    for (int st = 0; st < nst; st += DP) {
+#pragma unroll
+        for (int q = 0; q < DP; ++q) stage(q, st + q);
+    }
+
+#pragma unroll
+    for (int a = 0; a < AM; ++a) {
+        const int row = m0 + 16 * (AM * wm + a) + li;
+        if (row >= g.M) continue;
+#pragma unroll
+        for (int b = 0; b < AN; ++b) {
+            const int64_t at = (int64_t)row * g.ldy + n0 + 16 * (AN * wn + b) + 4 * gq;
+            if (!g.vec) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) store_out<EP>(g.y, at + r, acc[a][b][r]);
+                continue;
+            }
+            store_out4<EP>(g.y, at, acc[a][b]);
+        }
+    }
+}
+
+// ── dense fp16 weights, row-major ──
 //
 // y = epilogue(fp16(x · wᵀ)) for x [groups][M][lda] fp16 and w [N][K] fp16
-// (rows K-contiguous): the long pass once the weight is fp16 — a dense fp16
-// base, or a quantised one dequantised into a workspace (the quantised entry
-// points do that for shapes with many output tiles: one dequant per matrix
-// costs 10-35 µs against milliseconds of products at M ≥ 4096).
+// (rows K-contiguous): a dense fp16 base (rwkv_f16_gemm).
 //
 // A workgroup of 8 waves computes a 256 (input rows) × 256 (output features)
 // tile in stages of 64 columns.  Both operands are staged in LDS as rows of
@@ -407,13 +893,10 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
 // (sched_group_barrier): measured 0.42-0.51 of the fp16 peak at M = 8192
 // against 0.38-0.43 with them grouped.
 //
-// Per output the products and their order are the fused kernel's
-// (v_mfma_f32_16x16x32_f16 over the same 32-column units, first to last, the
-// same lane layout), so with w = the fp16 weight the fused kernel decodes,
-// the result is quant_gemm_kernel's bitwise.
+// Per output the products and their order are quant_gemm_kernel's
+// (v_mfma_f32_16x16x32_f16 over the same 32-column units, first to last), so
+// with w = the fp16 weight that kernel decodes, the result is its bitwise.
 constexpr int DT = 256;         // dense tile: input rows = output features
-constexpr int DKS = 64;         // columns per stage
-constexpr int DENSE_MIN_TILES = 128;   // dense route from this many 256 × 256 tiles
 
 struct DenseArgs {
     const _Float16* x;    // [groups][M][lda]
@@ -555,42 +1038,6 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(DenseArgs g) {
     }
 }
 
-// The K ranges of a split launch summed in range order (a fixed order: the
-// result does not depend on which workgroup finished first), then the
-// epilogue of the one-range kernel: fp16 rounding, store / add / relu².
-// Thread i takes 4 consecutive outputs of one row (N is a multiple of 128).
-template <int EP>
-__global__ __launch_bounds__(256) void gemm_split_reduce(const float* __restrict__ part, int S, int M, int N,
-                                                         void* y, int64_t ldy) {
-    const int64_t n4 = (int64_t)M * N / 4;
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n4) return;
-    const float4* p = reinterpret_cast<const float4*>(part) + i;
-    float4 a = p[0];
-    for (int k = 1; k < S; ++k) {
-        const float4 b = p[(int64_t)k * n4];
-        a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
-    }
-    const int64_t row = 4 * i / N, col = 4 * i % N;
-    const float v[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-    for (int c = 0; c < 4; ++c) store_out<EP>(y, row * ldy + col + c, v[c]);
-}
-
-// K ranges per launch: one where the (row block, feature block) tiles
-// already fill the chip; otherwise enough to reach about 384 workgroups
-// (two per CU hold 512), each range at least 3 stages of 64 columns.  A
-// tile's stages run one after another, each waiting on its loads (about
-// 2 µs a stage at a few workgroups per XCD), so few tiles over a long K
-// take K/64 such waits: 128 rows × 768 features × K 3072, 6 tiles, took
-// 100 µs in one range.
-int gemm_splits(int64_t M, int64_t N, int64_t K) {
-    const int64_t tiles = ((M + 127) / 128) * (N / 128);
-    if (tiles >= 160) return 1;
-    const int64_t want = (384 + tiles - 1) / tiles, most = K / BK / 3;
-    return (int)std::max<int64_t>(1, std::min(want, most));
-}
-
 // The dense kernel's shapes (x rows lda halves apart, group g at x + g·x_gstride).
 bool dense_shape_ok(int64_t M, int64_t OUT, int64_t IN, int64_t out_per, int64_t lda) {
     return M >= 1 && M <= ((int64_t)1 << 24) && OUT >= DT && OUT % DT == 0 && OUT <= ((int64_t)1 << 30) &&
@@ -599,19 +1046,80 @@ bool dense_shape_ok(int64_t M, int64_t OUT, int64_t IN, int64_t out_per, int64_t
            ((M + DT - 1) / DT) * (OUT / DT) < ((int64_t)1 << 31);
 }
 
-// The quantised entry points take the dense route (dequantise into the
-// workspace, then dense_gemm_kernel) from DENSE_MIN_TILES tiles: half a round
-// of the 256 CUs.  Below it the fused kernel's 128 × 128 tiles (and its K
-// split) keep more CUs busy and no dequant is paid: 4096 rows × 1024 × 1024
-// took 34 µs fused against 9.5 + 34 µs dequant + dense.
-bool dense_prefers(int64_t M, int64_t OUT, int64_t IN) {
-    return dense_shape_ok(M, OUT, IN, OUT, IN) && ((M + DT - 1) / DT) * (OUT / DT) >= DENSE_MIN_TILES;
+// Which kernel a quantised pass takes when the caller gave a workspace, by
+// shape alone: fp32 inputs take the same sums as fp16 ones (an input is
+// rounded to fp16 either way, so equal values give equal results).  Times in
+// µs, fitted to graph-timed calls on MI355X (sb6 4-bit, 4-4096 rows, 768-8192 ×
+// 768-4096 matrices; within ~20 %): a workgroup's time is a start plus its K,
+// and CUs take ceil(workgroups / 256) of them in turn.
+//   * Waves splitting K (gemm_ks_kernel): A + B·K/1024 per tile.  Against one
+//     fused launch with K ranges and their reduction: 128 rows × 3072 × 768
+//     6.5 (13.1), 128 × 768 × 3072 7.0 (16.1), 16 × 4096 × 4096 7.6 (22.8),
+//     512 × 1024 × 4096 18.2 (28.3).  Its weights are decoded once per row
+//     block, so many row blocks favour:
+//   * the dense route (dequant_tiles_kernel + dense_tiles_kernel): the dequant
+//     (a launch plus its bytes), then per 64-column stage the latency of one
+//     tile or the rate of a full CU.  Against the same: 1001 × 3072 × 1024
+//     21.7 (32.9), 2048 × 1024 × 4096 30.2 (61), 4096 × 1024 × 4096 44.7 (134);
+//     against a row-major weight through LDS 4096 × 4096 × 4096 119 (126).
+struct GemmRoute {
+    enum Kind { kFused, kSplitWaves, kDense } kind = kFused;
+    int mt = 0, nt = 0;   // kSplitWaves: the tile / 16 (fp16 inputs)
+    int waves = 0;
+    int tile = 0;         // kDense: the tile shape's id
+};
+
+GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, int64_t out_per, int64_t lda) {
+    const auto blocks = [&](int tm, int tn) { return (double)((M + tm - 1) / tm) * (double)(N / tn); };
+    const double k = (double)K / 1024, st = (double)K / DKS;
+    GemmRoute best;
+    double cost = 1e30;
+    struct Ks {
+        int mt, nt, waves, many;   // waves per workgroup: one round of the CUs, more
+        double a, b;
+    };
+    static const Ks ks[] = {{1, 1, 8, 8, 3.0, 0.95},  {2, 1, 12, 6, 3.3, 1.07}, {2, 2, 8, 8, 3.5, 1.8},
+                            {4, 1, 8, 4, 3.6, 1.75}, {4, 2, 7, 7, 3.9, 2.9},   {4, 4, 6, 6, 3.0, 6.8}};
+    for (const Ks& e : ks) {
+        // offsets within a tile's input rows are 32-bit
+        if ((int64_t)16 * e.mt * lda * 4 >= ((int64_t)1 << 31)) continue;
+        const double n = std::ceil(blocks(16 * e.mt, 16 * e.nt) / 256);
+        // 64 × 16 tiles of four waves share a CU past one round
+        const double c = 2 + n * (e.mt == 4 && e.nt == 1 && n > 1 ? 1.1 + 1.6 * k : e.a - 2 + e.b * k);
+        if (c >= cost) continue;
+        cost = c;
+        int w = n > 1 ? e.many : e.waves;
+        if (e.mt * e.nt == 1 && K >= 4096) w = 16;
+        w = (int)std::min<int64_t>(w, K / KS_COLS);
+        best = {GemmRoute::kSplitWaves, e.mt, e.nt, w, 0};
+    }
+    struct Tile {
+        int tm, tn, id;
+        double latency, rate;   // per stage: one tile alone, a tile on a full chip
+    };
+    static const Tile tiles[] = {
+        {64, 64, 64, 0.265, 0.21}, {64, 128, 128, 0.34, 0.34}, {128, 128, 256, 0.465, 0.52}, {256, 256, 512, 1.2, 1.7}};
+    for (const Tile& t : tiles) {
+        if (N % t.tn || out_per % t.tn || (int64_t)t.tm * lda * 4 >= ((int64_t)1 << 31) ||
+            (int64_t)t.tn * K * 2 >= ((int64_t)1 << 31))
+            continue;
+        const double n = blocks(t.tm, t.tn) / 256, whole = std::floor(n), part = n - whole;
+        const double per_stage = whole * t.rate + (part > 0 ? std::max(t.latency, t.rate * part) : 0.0);
+        const double c = 5.7 + (double)N * (double)K / 2.4e6 + st * per_stage;
+        if (c >= cost) continue;
+        cost = c;
+        best = {GemmRoute::kDense, 0, 0, 0, t.id};
+    }
+    return best;
 }
 
+// Bytes of workspace a pass of this shape takes: the dense route's fp16 weight.
+// The split over waves needs none of its own; it asks for two ranges' fp32
+// sums, the least that a caller's workspace for such a shape has held, so that
+// the size still tells which shapes want one.
 int64_t gemm_workspace(int64_t M, int64_t N, int64_t K) {
-    if (dense_prefers(M, N, K)) return N * K * 2;   // the fp16 weight
-    const int S = gemm_splits(M, N, K);
-    return S > 1 ? (int64_t)S * M * N * 4 : 0;
+    const GemmRoute r = gemm_route(M, N, K, N, K);
+    return r.kind == GemmRoute::kDense ? N * K * 2 : r.kind == GemmRoute::kSplitWaves ? 2 * M * N * 4 : 0;
 }
 
 template <int EP>
@@ -633,13 +1141,75 @@ void launch_dense(const DenseArgs& g, int epilogue, hipStream_t s) {
 // not hidden).
 template <class F, typename TA, int EP>
 void launch_gemm(const GemmArgs& g, hipStream_t s) {
-    const int64_t blocks = (int64_t)((g.M + 127) / 128) * (g.N / 128) * g.splits;
+    const int64_t blocks = (int64_t)((g.M + 127) / 128) * (g.N / 128);
     rwkv::launch(quant_gemm_kernel<F, TA, EP, 8, 2>, dim3((unsigned)blocks), dim3(256), s, g);
-    if (g.splits > 1) {
-        const int64_t n4 = (int64_t)g.M * g.N / 4;
-        rwkv::launch(gemm_split_reduce<EP>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), s, g.part, g.splits,
-                     g.M, g.N, g.y, g.ldy);
+}
+
+// y rows take aligned 4-wide accesses.
+bool vec_rows(const GemmArgs& g, int epilogue) {
+    return g.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(g.y) % (epilogue == 2 ? 8 : 16) == 0;
+}
+
+template <class F, typename TA, int MT, int NT, int MAXW>
+void launch_ks_tile(const KsArgs& a, int W, hipStream_t s) {
+    constexpr int BM = 16 * MT, BN = 16 * NT;
+    const int64_t blocks = (int64_t)((a.g.M + BM - 1) / BM) * (a.g.N / BN);
+    const size_t lds = (size_t)W * std::max(BM * (BN + KS_PAD) * 4, ks_wave_lds<F>(MT, NT));
+    rwkv::launch_lds(gemm_ks_kernel<F, TA, MT, NT, MAXW>, dim3((unsigned)blocks), dim3(64 * W), lds, s, a);
+}
+
+// The sums depend on the waves alone, not on the tile: fp32 inputs, whose
+// staging takes twice the registers, run the same waves on another tile.
+template <class F, typename TA>
+void launch_ks(const GemmArgs& g, const GemmRoute& r, int epilogue, hipStream_t s) {
+    const KsArgs a{g, epilogue, vec_rows(g, epilogue)};
+    const int t = 10 * r.mt + r.nt;
+    const int W = std::min<int>(r.waves, (int)(KS_LDS / ks_wave_lds<F>(r.mt, r.nt)));
+    if (t == 11) launch_ks_tile<F, TA, 1, 1, 16>(a, W, s);
+    else if (t == 21) launch_ks_tile<F, TA, 2, 1, 12>(a, W, s);
+    else if (t == 22) launch_ks_tile<F, TA, 2, 2, 8>(a, W, s);
+    else if constexpr (sizeof(TA) == 4) {
+        if (t == 41) launch_ks_tile<F, TA, 2, 2, 8>(a, W, s);
+        else launch_ks_tile<F, TA, 2, 4, 8>(a, W, s);
+    } else {
+        if (t == 41) launch_ks_tile<F, TA, 4, 1, 8>(a, W, s);
+        else if (t == 42) launch_ks_tile<F, TA, 4, 2, 8>(a, W, s);
+        else launch_ks_tile<F, TA, 4, 4, 8>(a, W, s);
     }
+}
+
+template <typename TA, int EP, int WM, int WN, int AM, int AN, int DP, int DA>
+void launch_tiles_shape(const DenseTArgs& g, hipStream_t s) {
+    constexpr int TM = 16 * WM * AM, TN = 16 * WN * AN;
+    rwkv::launch(dense_tiles_kernel<TA, EP, WM, WN, AM, AN, DP, DA>,
+                 dim3((unsigned)((int64_t)((g.M + TM - 1) / TM) * (g.N / TN))), dim3(64 * WM * WN), s, g);
+}
+
+template <typename TA, int EP>
+void launch_tiles_ep(const DenseTArgs& g, int tile, hipStream_t s) {
+    switch (tile) {
+        case 64: launch_tiles_shape<TA, EP, 1, 4, 4, 1, 4, 4>(g, s); break;     // 64 × 64
+        case 128: launch_tiles_shape<TA, EP, 1, 4, 4, 2, 4, 2>(g, s); break;    // 64 × 128
+        case 256: launch_tiles_shape<TA, EP, 1, 4, 8, 2, 4, sizeof(TA) == 2 ? 2 : 1>(g, s); break;    // 128 × 128
+        default: launch_tiles_shape<TA, EP, 2, 4, 8, 4, 2, 1>(g, s); break;     // 256 × 256
+    }
+}
+
+template <typename TA>
+void launch_tiles_ta(const DenseTArgs& a, int tile, int epilogue, hipStream_t s) {
+    if (epilogue == 0) launch_tiles_ep<TA, 0>(a, tile, s);
+    else if (epilogue == 1) launch_tiles_ep<TA, 1>(a, tile, s);
+    else launch_tiles_ep<TA, 2>(a, tile, s);
+}
+
+// The dense route: dequantise into the workspace (operand order), then multiply.
+template <class F>
+void launch_tiles(const GemmArgs& g, int tile, bool f16, void* workspace, int epilogue, hipStream_t s) {
+    _Float16* w = reinterpret_cast<_Float16*>(workspace);
+    const int64_t waves = (int64_t)(g.N / 16) * (g.K / 128);
+    rwkv::launch(dequant_tiles_kernel<F>, dim3((unsigned)((waves + 3) / 4)), dim3(256), s, g, w);
+    const DenseTArgs a{g.x, g.lda, g.x_gstride, w, g.y, g.ldy, g.M, g.N, g.K, g.out_per, vec_rows(g, epilogue)};
+    f16 ? launch_tiles_ta<_Float16>(a, tile, epilogue, s) : launch_tiles_ta<float>(a, tile, epilogue, s);
 }
 
 template <class F>
@@ -649,6 +1219,14 @@ void launch_gemm_ep(const GemmArgs& g, bool f16, int epilogue, hipStream_t s) {
         case 1: f16 ? launch_gemm<F, _Float16, 1>(g, s) : launch_gemm<F, float, 1>(g, s); break;
         default: f16 ? launch_gemm<F, _Float16, 2>(g, s) : launch_gemm<F, float, 2>(g, s); break;
     }
+}
+
+template <class F>
+void launch_routed(const GemmArgs& g, const GemmRoute& r, bool f16, void* workspace, int epilogue, hipStream_t s) {
+    if (r.kind == GemmRoute::kDense) launch_tiles<F>(g, r.tile, f16, workspace, epilogue, s);
+    else if (r.kind == GemmRoute::kSplitWaves)
+        f16 ? launch_ks<F, _Float16>(g, r, epilogue, s) : launch_ks<F, float>(g, r, epilogue, s);
+    else launch_gemm_ep<F>(g, f16, epilogue, s);
 }
 
 bool gemm_shape_ok(int64_t OUT, int64_t IN, int64_t out_per) {
@@ -688,25 +1266,6 @@ rwkv_status gemm_workspace_check(const char* who, int64_t M, int64_t N, int64_t 
     return RWKV_OK;
 }
 
-// The dense route of a quantised entry point: fp16 inputs, a workspace, and
-// a shape the dense kernel takes with enough tiles.
-bool take_dense(rwkv_dtype x_dt, int64_t M, int64_t OUT, int64_t IN, int64_t out_per, int64_t lda,
-                const void* workspace) {
-    return workspace != nullptr && x_dt == RWKV_F16 && dense_prefers(M, OUT, IN) &&
-           dense_shape_ok(M, OUT, IN, out_per, lda);
-}
-
-// The fused launch's K ranges: several where the shape asks for them and the
-// caller passed a workspace, one otherwise.
-void gemm_split_args(GemmArgs& g, void* workspace) {
-    g.part = nullptr;
-    g.splits = 1;
-    const int S = gemm_splits(g.M, g.N, g.K);
-    if (workspace == nullptr || S == 1 || dense_prefers(g.M, g.N, g.K)) return;
-    g.part = reinterpret_cast<float*>(workspace);
-    g.splits = S;
-}
-
 }  // namespace
 
 extern "C" {
@@ -733,21 +1292,14 @@ rwkv_status rwkv_sb6_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda
     c = gemm_workspace_check("sb6_gemm", M, OUT, IN, workspace, workspace_bytes);
     if (c != RWKV_OK) return c;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (take_dense(x_dt, M, OUT, IN, out_per, lda, workspace)) {
-        c = rwkv_sb6_dequant(qblk, qsqm, ddm, workspace, RWKV_F16, OUT, IN, xbits, stream);
-        if (c != RWKV_OK) return c;
-        launch_dense(DenseArgs{reinterpret_cast<const _Float16*>(x), lda, x_group_stride,
-                               reinterpret_cast<const _Float16*>(workspace), y, ldy, (int)M, (int)OUT, (int)IN,
-                               (int)out_per},
-                     epilogue, s);
-    } else {
-        GemmArgs g{x, lda, x_group_stride, qblk, qsqm, ddm, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per};
-        gemm_split_args(g, workspace);
-        const bool f16 = x_dt == RWKV_F16;
-        if (xbits == 0) launch_gemm_ep<Sb6W<0>>(g, f16, epilogue, s);
-        else if (xbits == 1) launch_gemm_ep<Sb6W<1>>(g, f16, epilogue, s);
-        else launch_gemm_ep<Sb6W<2>>(g, f16, epilogue, s);
-    }
+    GemmArgs g{x, lda, x_group_stride, qblk, qsqm, ddm, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per};
+    const bool f16 = x_dt == RWKV_F16;
+    // one K range without a workspace
+    const GemmRoute r = workspace ? gemm_route(M, OUT, IN, out_per, lda) : GemmRoute{};
+    if (r.kind == GemmRoute::kDense) rwkv::counters().sb6_dequant.fetch_add(1);
+    if (xbits == 0) launch_routed<Sb6W<0>>(g, r, f16, workspace, epilogue, s);
+    else if (xbits == 1) launch_routed<Sb6W<1>>(g, r, f16, workspace, epilogue, s);
+    else launch_routed<Sb6W<2>>(g, r, f16, workspace, epilogue, s);
     RWKV_REQUIRE(hipGetLastError() == hipSuccess, RWKV_E_HIP, "sb6_gemm: launch failed");
     rwkv::counters().sb6_gemm.fetch_add(1);
     rwkv::clear_error();
@@ -771,20 +1323,13 @@ rwkv_status rwkv_sym_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda
     c = gemm_workspace_check("sym_gemm", M, OUT, IN, workspace, workspace_bytes);
     if (c != RWKV_OK) return c;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (take_dense(x_dt, M, OUT, IN, out_per, lda, workspace)) {
-        c = rwkv_sym_dequant(qblk, qs, d, workspace, RWKV_F16, OUT, IN, bits, stream);
-        if (c != RWKV_OK) return c;
-        launch_dense(DenseArgs{reinterpret_cast<const _Float16*>(x), lda, x_group_stride,
-                               reinterpret_cast<const _Float16*>(workspace), y, ldy, (int)M, (int)OUT, (int)IN,
-                               (int)out_per},
-                     epilogue, s);
-    } else {
-        GemmArgs g{x, lda, x_group_stride, qblk, qs, d, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per};
-        gemm_split_args(g, workspace);
-        const bool f16 = x_dt == RWKV_F16;
-        if (bits == 8) launch_gemm_ep<SymW<8>>(g, f16, epilogue, s);
-        else launch_gemm_ep<SymW<6>>(g, f16, epilogue, s);
-    }
+    GemmArgs g{x, lda, x_group_stride, qblk, qs, d, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per};
+    const bool f16 = x_dt == RWKV_F16;
+    // one K range without a workspace
+    const GemmRoute r = workspace ? gemm_route(M, OUT, IN, out_per, lda) : GemmRoute{};
+    if (r.kind == GemmRoute::kDense) rwkv::counters().sym_dequant.fetch_add(1);
+    if (bits == 8) launch_routed<SymW<8>>(g, r, f16, workspace, epilogue, s);
+    else launch_routed<SymW<6>>(g, r, f16, workspace, epilogue, s);
     RWKV_REQUIRE(hipGetLastError() == hipSuccess, RWKV_E_HIP, "sym_gemm: launch failed");
     rwkv::counters().sym_gemm.fetch_add(1);
     rwkv::clear_error();

@@ -560,8 +560,8 @@ _GEMM_EP = {"store": 0, "add": 1, "relu2_f16": 2}
 
 
 def rwkvq_gemm_workspace(rows: int, out_features: int, in_features: int) -> int:
-    """Bytes of the workspace a long-pass GEMM of this shape splits its K sum
-    with (0: the shape runs as one range)."""
+    """Bytes of the workspace a long-pass GEMM of this shape wants (0: it runs as
+    one K range without; the C entry runs any shape so when given none)."""
     return int(_lib.lib().rwkv_quant_gemm_workspace(rows, out_features, in_features))
 
 
@@ -601,8 +601,9 @@ def rwkvq_sb6_gemm(x, qblk, qsqm, ddm, out_features: int, in_features: int, xbit
     [M, OUT] = fp16(fp16(x)·fp16(W)ᵀ) with fp32 sums.  x [M, IN] (one matrix)
     or [G, M, IN] (G = OUT / out_per row-concatenated matrices, matrix g
     reading x[g]), fp32 or fp16.  epilogue "store" / "add" (fp32 `out`, added
-    into) / "relu2_f16" (relu(·)² in an fp16 `out`).  `split`: shapes with few
-    output tiles sum K in ranges (a workspace per call; False: one range)."""
+    into) / "relu2_f16" (relu(·)² in an fp16 `out`).  `split`: take the kernels
+    that want a workspace (one per call), some of which sum K in ranges (False:
+    one range)."""
     per = out_features if out_per is None else out_per
     if not rwkvq_sb6_gemm_applies(out_features, in_features, xbits, per):
         raise ValueError(f"sb6 GEMM: [{out_features}, {in_features}] xbits={xbits} out_per={per} not taken")

@@ -1,0 +1,77 @@
+"""The kernels a quantised long pass is routed to by its shape (csrc/gemm.hip, gemm_route): the K sum split over a
+workgroup's waves, on every tile, and the dense route over operand-ordered weights, on every tile.
+
+Each shape: fp16 and fp32 inputs of equal values give equal bits; every output is the fp16 rounding of the exact
+(float64) sum of the fp16 operands up to ½ fp16 ulp + 2^-16·Σ|x·w| (an fp32 sum's rounding); an output with a row
+stride that rules out wide stores gets the same values and leaves its other columns alone."""
+import numpy as np
+import pytest
+import torch
+
+from swiftrwkv_amd import _lib, quant as Q
+from tests.test_gpu_prefill import check_f16_rounding
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# (rows, OUT, IN, groups): one shape or more per tile, with partial row blocks, one row, a single K step per wave,
+# uneven steps per wave, more steps than one block of scale words
+SHAPES = [
+    (1, 256, 256, 1), (17, 128, 512, 1), (16, 768, 5376, 1),          # 16 × 16
+    (33, 3072, 768, 1), (31, 1536, 2304, 3),                          # 32 × 16
+    (65, 2048, 1536, 1), (150, 1536, 512, 3),                         # 32 × 32
+    (130, 1024, 4096, 1),                                             # 64 × 16
+    (129, 2304, 768, 1), (90, 4096, 2304, 1),                         # 64 × 32
+    (257, 2304, 512, 1), (700, 768, 1024, 1),                         # 64 × 64
+    (1300, 512, 2048, 1),                                             # dense 64 × 64
+    (700, 2304, 768, 3), (1030, 1024, 1280, 1),                       # dense 64 × 128
+    (1001, 3072, 1024, 3), (1500, 2304, 256, 1),                      # dense 128 × 128
+    (1999, 4608, 512, 1),                                             # dense 256 × 256
+]
+
+
+def matrix(fmt, OUT, IN, seed):
+    """(loader buffers, the gemm of them, C entry, code bits, their fp16 weight) of a Gaussian matrix."""
+    kind, bits = fmt.split(":")
+    bits = int(bits)
+    w = np.random.default_rng(seed).standard_normal((OUT, IN), dtype=np.float32) * np.float32(0.05)
+    L = _lib.lib()
+    if kind == "sb6":
+        d = Q.encode_sb6(w, 4 + bits)
+        qblk, qsqm, ddm, xb = Q.rwkvq_sb6_to_k3(d["codes_packed"], d["gw_qsqm"], d["gw_d"], d["gw_dm"], d.get("gw_qh"),
+                                                d.get("gw_qh2"), (OUT, IN))
+        assert xb == bits
+        bufs = [torch.from_numpy(z).to(DEV) for z in (qblk, qsqm, ddm.view(np.float16))]
+        return bufs, Q.rwkvq_sb6_gemm, L.rwkv_sb6_gemm, bits, Q.rwkvq_dequant_dense(*bufs, OUT, IN, 8, bits, torch.float16)
+    d = Q.encode_sym(w, bits)
+    codes = d["codes"].view(np.uint8) if bits == 8 else Q.rwkvq_sym_interleave(d["codes_packed"], d["gw_qh"], d["gw_qh2"],
+                                                                               (OUT, IN))
+    bufs = [torch.from_numpy(z).to(DEV) for z in (codes, d["gw_qs"].view(np.uint8), d["gw_d"])]
+    return bufs, Q.rwkvq_sym_gemm, L.rwkv_sym_gemm, bits, Q.rwkvq_dequant_sym(*bufs, OUT, IN, bits, torch.float16)
+
+
+@pytest.mark.parametrize("fmt", ["sb6:0", "sb6:1", "sb6:2", "sym:8", "sym:6"])
+@pytest.mark.parametrize("M,OUT,IN,G", SHAPES)
+def test_quant_gemm_routes(fmt, M, OUT, IN, G):
+    print(f"[case] gemm route {fmt} M={M} {OUT}x{IN} G={G}", flush=True)
+    bufs, gemm, entry, bits, w16 = matrix(fmt, OUT, IN, M + OUT)
+    per = OUT // G
+    gen = torch.Generator(device=DEV).manual_seed(M + IN)
+    x = torch.randn((G, M, IN), generator=gen, device=DEV).half()
+    y = gemm(x, *bufs, OUT, IN, bits, out_per=per)
+    assert torch.equal(gemm(x.float(), *bufs, OUT, IN, bits, out_per=per), y)
+    rows = slice(0, M) if M < 300 else torch.tensor([*range(40), *range(M - 40, M)], device=DEV)
+    for g in range(G):
+        xs, ws = x[g][rows].double(), w16[g * per:(g + 1) * per].double()
+        got = y[rows][:, g * per:(g + 1) * per]
+        check_f16_rounding(got.cpu().numpy(), (xs @ ws.T).cpu().numpy(), (xs.abs() @ ws.abs().T).cpu().numpy())
+    h = gemm(x, *bufs, OUT, IN, bits, out_per=per, epilogue="relu2_f16")
+    assert torch.equal(h, (torch.relu(y) * torch.relu(y)).half())
+    base = torch.randn((M, OUT + 3), generator=gen, device=DEV)
+    out = base.clone()
+    need = Q.rwkvq_gemm_workspace(M, OUT, IN)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    _lib.check(entry(x.data_ptr(), _lib.F16, M, IN, M * IN, *[b.data_ptr() for b in bufs], out.data_ptr(), OUT + 3, OUT,
+                     IN, bits, per, 1, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out[:, :OUT], base[:, :OUT] + y)
+    assert torch.equal(out[:, OUT:], base[:, OUT:])

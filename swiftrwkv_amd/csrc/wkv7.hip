@@ -21,17 +21,16 @@
 // construction (the reference's invariants WKV7SequenceTests,
 // WKV7StateTests.swift:178-186, DecodeKernelTests.swift:27-39).
 //
-// Backward (column-owned, the scheme of ckptBwdKernelV2,
-// WKV7Train.swift:234-339).  Eight waves per head: lane i owns key column i,
-// wave q owns value rows J_q = [8q, 8q+8).  Instead of reconstructing earlier
-// states by dividing by w (which re-amplifies the forward's rounding by up to
-// 1/w^15), each 16-step chunk's states are recomputed forward from the
-// previous checkpoint (or h_in) with the stored sa and the forward kernel's
-// exact FMA sequence, so they are bitwise the forward's states.  The chunk is
-// handled as two 8-step windows whose states are held in registers.  Step
-// vectors are staged per chunk in LDS (coalesced loads issued one chunk
-// ahead); dsa is the one quantity exchanged inside a step (one barrier per
-// step); every output is summed over the eight waves from an LDS ring.
+// Backward (the results of ckptBwdKernelV2, WKV7Train.swift:234-339).  Eight
+// waves per head; wave q owns the value rows [8q, 8q+8) of the states and of
+// dS, and the key columns [8q, 8q+8) of a second copy of dS.  Instead of
+// reconstructing earlier states by dividing by w (which re-amplifies the
+// forward's rounding by up to 1/w^15), each 16-step chunk's states are
+// recomputed forward from the previous checkpoint (or h_in) with the stored sa
+// in the forward's order of operations, and held in registers.  Step vectors
+// are staged per chunk in LDS (coalesced loads issued one chunk ahead); dsa is
+// the one quantity exchanged inside a step (one barrier per step); every
+// output is summed over the eight waves from an LDS ring.
 // Variant 1 is the reference's row-owned ckptBwdKernel (WKV7Train.swift:
 // 99-205), which does divide by w: wkv7_bwd_rows_kernel below.
 //
@@ -64,14 +63,16 @@ __device__ __forceinline__ void store1(void* __restrict__ p, int64_t off, float 
     if constexpr (DT == RWKV_F32) {
         reinterpret_cast<float*>(p)[off] = x;
     } else if constexpr (DT == RWKV_BF16) {
-        uint32_t u = __float_as_uint(x);
-        uint16_t h;
-        if ((u & 0x7f800000u) == 0x7f800000u && (u & 0x7fffffu)) h = (uint16_t)((u >> 16) | 0x40u);
-        else h = (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-        reinterpret_cast<uint16_t*>(p)[off] = h;
+        reinterpret_cast<uint16_t*>(p)[off] = __builtin_bit_cast(uint16_t, (__bf16)x);
     } else {
         reinterpret_cast<uint16_t*>(p)[off] = __builtin_bit_cast(uint16_t, (_Float16)x);
     }
+}
+
+// Element off of p.
+template <int DT>
+__device__ __forceinline__ const void* at(const void* p, int64_t off) {
+    return reinterpret_cast<const char*>(p) + off * (DT == RWKV_F32 ? 4 : 2);
 }
 
 // ─────────────────────────────── forward ───────────────────────────────
@@ -356,75 +357,88 @@ __global__ __launch_bounds__(64) void wkv7_fwd4_kernel(
 
 // ─────────────────────────────── backward ───────────────────────────────
 constexpr int BQ = 8;     // waves per head
-constexpr int BJ = 8;     // value rows per wave
 constexpr int NVEC = 8;   // staged step vectors: r w k v a b dy sa
 constexpr int NOUT = 6;   // dr dw dk db dv da
-constexpr int WIN = 8;    // steps per register window (two per chunk)
-
-#define RWKV_BC8(n) RWKV_BC(n)
-
-// 8-wide broadcast helpers: lane l holds element 8q + (l & 7) of a step vector
-// over the wave's rows; row_newbcast:jj reads row jj of the wave's block.
-// (1) recompute: n_jj = v_j·k_i ; n_jj += sa_j·b_i      (then n += w_i·S in C++)
-#define RWKV_RC(jj) \
-    "v_mul_f32_dpp %[n" #jj "], %[V], %[ki]" RWKV_BC(jj) "v_fmac_f32_dpp %[n" #jj "], %[SA], %[bi]" RWKV_BC(jj)
-__device__ __forceinline__ void bwd_recompute8(const float (&S)[BJ], float (&N)[BJ], float V, float SA, float ki,
-                                               float bi, float wi) {
-    asm("s_nop 1\n\t" RWKV_RC(0) RWKV_RC(1) RWKV_RC(2) RWKV_RC(3) RWKV_RC(4) RWKV_RC(5) RWKV_RC(6) RWKV_RC(7)
-        : [n0] "=&v"(N[0]), [n1] "=&v"(N[1]), [n2] "=&v"(N[2]), [n3] "=&v"(N[3]), [n4] "=&v"(N[4]),
-          [n5] "=&v"(N[5]), [n6] "=&v"(N[6]), [n7] "=&v"(N[7])
-        : [V] "v"(V), [SA] "v"(SA), [ki] "v"(ki), [bi] "v"(bi));
-#pragma unroll
-    for (int jj = 0; jj < BJ; ++jj) N[jj] = fmaf(wi, S[jj], N[jj]);
-}
-
-// (2) first half of a reverse step, 4 rows at a time:
-//   dr += dy_j·S_j ; dT_j += dy_j·r_i ; dR_j += r_j·dy_i
-#define RWKV_B1(jj, e)                                              \
-    "v_fmac_f32_dpp %[dr], %[DY], %[sa" #e "]" RWKV_BC(jj)          \
-    "v_fmac_f32_dpp %[t" #e "], %[DY], %[ri]" RWKV_BC(jj)           \
-    "v_fmac_f32_dpp %[u" #e "], %[R], %[dyi]" RWKV_BC(jj)
-#define RWKV_B1_BLOCK(j0, j1, j2, j3, o)                                                                  \
-    asm("s_nop 1\n\t" RWKV_B1(j0, 0) RWKV_B1(j1, 1) RWKV_B1(j2, 2) RWKV_B1(j3, 3)                          \
-        : [dr] "+v"(pdr), [t0] "+v"(dT[o]), [t1] "+v"(dT[o + 1]), [t2] "+v"(dT[o + 2]), [t3] "+v"(dT[o + 3]), \
-          [u0] "+v"(dR[o]), [u1] "+v"(dR[o + 1]), [u2] "+v"(dR[o + 2]), [u3] "+v"(dR[o + 3])               \
-        : [sa0] "v"(Sa[o]), [sa1] "v"(Sa[o + 1]), [sa2] "v"(Sa[o + 2]), [sa3] "v"(Sa[o + 3]), [DY] "v"(DY),  \
-          [R] "v"(R), [ri] "v"(ri), [dyi] "v"(dyi))
-// (3) dk += v_j·dT_j ; db += sa_j·dT_j ; dv += k_j·dR_j ; dsa += b_j·dR_j
-#define RWKV_B2(jj, e)                                              \
-    "v_fmac_f32_dpp %[dk], %[V], %[t" #e "]" RWKV_BC(jj)            \
-    "v_fmac_f32_dpp %[db], %[SA], %[t" #e "]" RWKV_BC(jj)           \
-    "v_fmac_f32_dpp %[dv], %[K], %[u" #e "]" RWKV_BC(jj)            \
-    "v_fmac_f32_dpp %[ds], %[B], %[u" #e "]" RWKV_BC(jj)
-#define RWKV_B2_BLOCK(j0, j1, j2, j3, o)                                                                  \
-    asm("s_nop 1\n\t" RWKV_B2(j0, 0) RWKV_B2(j1, 1) RWKV_B2(j2, 2) RWKV_B2(j3, 3)                          \
-        : [dk] "+v"(pdk), [db] "+v"(pdb), [dv] "+v"(pdv), [ds] "+v"(pds)                                   \
-        : [t0] "v"(dT[o]), [t1] "v"(dT[o + 1]), [t2] "v"(dT[o + 2]), [t3] "v"(dT[o + 3]), [u0] "v"(dR[o]),    \
-          [u1] "v"(dR[o + 1]), [u2] "v"(dR[o + 2]), [u3] "v"(dR[o + 3]), [V] "v"(V), [SA] "v"(SA), [K] "v"(K), \
-          [B] "v"(B))
-// (4) da += dsa_j·Sp_j ; dR_j ← a_j·dsa_i + w_j·dR_j ; dT_j ← dsa_j·a_i (+ w_i·dT_j in C++)
-#define RWKV_B3(jj, e)                                              \
-    "v_fmac_f32_dpp %[da], %[DS], %[sp" #e "]" RWKV_BC(jj)          \
-    "v_mul_f32_dpp %[nu" #e "], %[A], %[dsi]" RWKV_BC(jj)           \
-    "v_fmac_f32_dpp %[nu" #e "], %[W], %[u" #e "]" RWKV_BC(jj)      \
-    "v_mul_f32_dpp %[nt" #e "], %[DS], %[ai]" RWKV_BC(jj)
-#define RWKV_B3_BLOCK(j0, j1, j2, j3, o)                                                                      \
-    asm("s_nop 1\n\t" RWKV_B3(j0, 0) RWKV_B3(j1, 1) RWKV_B3(j2, 2) RWKV_B3(j3, 3)                              \
-        : [da] "+v"(pda), [nu0] "=&v"(nR[o]), [nu1] "=&v"(nR[o + 1]), [nu2] "=&v"(nR[o + 2]),                  \
-          [nu3] "=&v"(nR[o + 3]), [nt0] "=&v"(nT[o]), [nt1] "=&v"(nT[o + 1]), [nt2] "=&v"(nT[o + 2]),           \
-          [nt3] "=&v"(nT[o + 3])                                                                               \
-        : [sp0] "v"(Sp[o]), [sp1] "v"(Sp[o + 1]), [sp2] "v"(Sp[o + 2]), [sp3] "v"(Sp[o + 3]), [u0] "v"(dR[o]), \
-          [u1] "v"(dR[o + 1]), [u2] "v"(dR[o + 2]), [u3] "v"(dR[o + 3]), [DS] "v"(DS), [A] "v"(A), [W] "v"(W),  \
-          [dsi] "v"(dsa_i), [ai] "v"(ai))
-
-// Σ over the 8 waves' partials p[0..7] of one column (stride D floats), pairwise.
-__device__ __forceinline__ float sum8(const float* p) {
-    const float x0 = p[0], x1 = p[D], x2 = p[2 * D], x3 = p[3 * D];
-    const float x4 = p[4 * D], x5 = p[5 * D], x6 = p[6 * D], x7 = p[7 * D];
-    return ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7));
-}
 
 // Variant 2, the default.
+//
+// Eight waves per head.  Wave q holds the value rows 8q .. 8q + 7 of the state
+// S and of dS (lane = key column), and the key columns 8q .. 8q + 7 of a second
+// copy of dS (lane = value row): every sum is then a sum over registers, of the
+// wave's eight rows or columns, and the waves' partials meet in LDS — dsa = dS·b
+// in every step (the recurrence; one barrier per step), the six outputs a step
+// later.  Lane l stands for element (l + 8q) mod 64, so lanes 0 .. 7 hold the
+// wave's own rows' values of every step vector.
+//
+// The rank-1 updates and the sums over rows run on v_mfma_f32_4x4x1_16b_f32:
+// its A operand, four lanes broadcast to all (cbsz 4), is four rows' values,
+// its B operand 64 lanes.  One instruction (8 cycles) adds a row value ⊗ 64
+// columns to four registers, twice the vector ALU's rate, or one register's
+// share to two weighted sums, at its rate.  The fp32 matrix operations and the
+// vector ALU do not run side by side, and changing between them costs about
+// ten cycles, so a step keeps them in two groups (the scheduling barriers).
+// A chunk's 17 states are in registers (136 of 234), computed once: two windows
+// of eight steps repeat half of them.
+//
+// What bounds it: with 256 heads, one per CU, the issue of both waves of a SIMD
+// (the loads' and the barrier's latencies are hidden: loading the next step's
+// vectors early changes nothing).  8 × 4096 × 32 heads, bf16: 3.9 ms with the
+// vector ALU alone, whose products all take a broadcast operand, 3.0 ms so.  Four waves
+// of 16 rows (one per SIMD, half the LDS traffic): 4.7 ms.
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+
+// c + a[4·BLK .. 4·BLK + 3] ⊗ b: register r, lane l: lane 4·BLK + r of `a` times b's lane l.
+template <int BLK>
+__device__ __forceinline__ f32x4 outer4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 4, BLK, 0);
+}
+// A matrix's eight rows (or columns) of the wave as registers.
+struct Rows8 {
+    f32x4 lo, hi;
+};
+__device__ __forceinline__ Rows8 outer8(float a, float b, const Rows8& c) {
+    return {outer4<0>(a, b, c.lo), outer4<1>(a, b, c.hi)};
+}
+// Σ_j X0[j]·M_j and Σ_j X1[j]·M_j: X's lane 2j + x holds X_x[j].
+struct Pair {
+    float x0, x1;
+};
+__device__ __forceinline__ Pair dots8(float X, const Rows8& M) {
+    f32x4 e = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f};
+    e = outer4<0>(X, M.lo[0], e);
+    o = outer4<0>(X, M.lo[1], o);
+    e = outer4<1>(X, M.lo[2], e);
+    o = outer4<1>(X, M.lo[3], o);
+    e = outer4<2>(X, M.hi[0], e);
+    o = outer4<2>(X, M.hi[1], o);
+    e = outer4<3>(X, M.hi[2], e);
+    o = outer4<3>(X, M.hi[3], o);
+    return {e[0] + o[2], e[1] + o[3]};
+}
+
+// W_j·M_j, W's lane ≡ j (mod 8) of every 16-lane row (not inline assembly: the
+// compiler places the wait between the matrix cores' write of M and this read).
+template <int J>
+__device__ __forceinline__ float bcast(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + J, 0xf, 0xf, true));
+}
+__device__ __forceinline__ Rows8 scale8(float W, const Rows8& M) {
+    return {{bcast<0>(W) * M.lo[0], bcast<1>(W) * M.lo[1], bcast<2>(W) * M.lo[2], bcast<3>(W) * M.lo[3]},
+            {bcast<4>(W) * M.hi[0], bcast<5>(W) * M.hi[1], bcast<6>(W) * M.hi[2], bcast<7>(W) * M.hi[3]}};
+}
+
+// The 8 waves' partials of one element (stride D floats), and their sum, pairwise.
+struct Parts {
+    float x[8];
+    __device__ __forceinline__ explicit Parts(const float* p) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = p[i * D];
+    }
+    __device__ __forceinline__ float sum() const {
+        return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+    }
+};
+
 template <int DT, int GT>
 __global__ __launch_bounds__(512) void wkv7_bwd_kernel(
     const void* __restrict__ r, const void* __restrict__ w, const void* __restrict__ k,
@@ -434,185 +448,150 @@ __global__ __launch_bounds__(512) void wkv7_bwd_kernel(
     void* __restrict__ g_dw, void* __restrict__ g_dk, void* __restrict__ g_dv, void* __restrict__ g_da,
     void* __restrict__ g_db, float* __restrict__ dh_in, int T, int H) {
     __shared__ float stage[2][NVEC][CH][D];        // step vectors of a chunk, fp32
-    // Per-wave partials, column-contiguous so a wave's 64 lanes write 64
-    // consecutive words (no bank conflicts); summed over the 8 waves per column.
-    __shared__ float dsa_part[2][BQ][D];           // [parity][wave][column]
-    __shared__ float ring[3][NOUT][BQ][D];         // output partials of the last steps
+    __shared__ float dsa_part[2][BQ][D];           // [parity][wave][row]
+    __shared__ float ring[4][NOUT][BQ][D];         // output partials of the last steps
 
     const int tid = threadIdx.x;
-    const int i = tid & 63;                                    // key column
-    const int q = __builtin_amdgcn_readfirstlane(tid >> 6);    // value rows 8q .. 8q+7
-    const int jl = 8 * q + (i & 7);                            // row this lane broadcasts
+    const int l = tid & 63;
+    const int q = __builtin_amdgcn_readfirstlane(tid >> 6);    // rows (columns) 8q .. 8q+7
+    const uint32_t e = (l + 8 * q) & 63;                       // the lane's element
+    const int jw = 8 * q + (l & 7);                            // scale8's row
+    const int jx = 8 * q + ((l >> 1) & 7);                     // dots8's row
+    const bool odd = l & 1;
     const int bh = blockIdx.x;
     const int bi = bh / H, hi = bh - bi * H;
     const int64_t strideT = (int64_t)H * D;
     const int64_t base0 = ((int64_t)bi * T * H + hi) * D;
     const int64_t hb = (int64_t)bh * D * D;
     const int NC = T / CH;
-    const void* const vec_src[6] = {r, w, k, v, a, b};
-    void* const outs[NOUT] = {g_dr, g_dw, g_dk, g_db, g_dv, g_da};
 
     // chunk staging: thread covers 16 floats of the chunk's 8 × 16 × 64 block
     float stg[16];
+    const uint32_t so = (uint32_t)((tid >> 6) * strideT + l), so8 = (uint32_t)(8 * strideT);
     auto stage_load = [&](int c) {
+        const int64_t off = base0 + c * CH * strideT;
 #pragma unroll
-        for (int m = 0; m < 16; ++m) {
-            const int idx = tid + 512 * m;            // (vec, step, elem)
-            const int vi = idx >> 10, st = (idx >> 6) & 15, e = idx & 63;
-            const int64_t off = base0 + (int64_t)(c * CH + st) * strideT + e;
-            if (vi < 6) {
-                switch (vi) {
-                    case 0: stg[m] = load1<DT>(r, off); break;
-                    case 1: stg[m] = load1<DT>(w, off); break;
-                    case 2: stg[m] = load1<DT>(k, off); break;
-                    case 3: stg[m] = load1<DT>(v, off); break;
-                    case 4: stg[m] = load1<DT>(a, off); break;
-                    default: stg[m] = load1<DT>(b, off); break;
-                }
-            } else {
-                stg[m] = (vi == 6 ? dout : sa)[off];
+        for (int m = 0; m < 16; ++m) {   // vector m / 2, step 8·(m % 2) + wave
+            const uint32_t o = so + (m & 1) * so8;
+            switch (m >> 1) {
+                case 0: stg[m] = load1<DT>(at<DT>(r, off), o); break;
+                case 1: stg[m] = load1<DT>(at<DT>(w, off), o); break;
+                case 2: stg[m] = load1<DT>(at<DT>(k, off), o); break;
+                case 3: stg[m] = load1<DT>(at<DT>(v, off), o); break;
+                case 4: stg[m] = load1<DT>(at<DT>(a, off), o); break;
+                case 5: stg[m] = load1<DT>(at<DT>(b, off), o); break;
+                case 6: stg[m] = (dout + off)[o]; break;
+                default: stg[m] = (sa + off)[o];
             }
         }
     };
     auto stage_store = [&](int c) {
 #pragma unroll
-        for (int m = 0; m < 16; ++m) {
-            const int idx = tid + 512 * m;
-            stage[c & 1][idx >> 10][(idx >> 6) & 15][idx & 63] = stg[m];
-        }
+        for (int m = 0; m < 16; ++m) stage[c & 1][m >> 1][8 * (m & 1) + (tid >> 6)][l] = stg[m];
     };
-    (void)vec_src;
 
-    float dT[BJ], dR[BJ];   // dS[J_q, i] (column copy) and dS[i, J_q] (row copy)
+    Rows8 dT, dR;   // dS[8q + j, e] and dS[e, 8q + j]
+    const Rows8 zero = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    dT = dR = zero;
     if (dhout) {
 #pragma unroll
-        for (int jj = 0; jj < BJ; ++jj) dT[jj] = dhout[hb + (int64_t)(8 * q + jj) * D + i];
-        const float4* src = reinterpret_cast<const float4*>(dhout + hb + (int64_t)i * D + 8 * q);
-        const float4 f0 = src[0], f1 = src[1];
-        dR[0] = f0.x; dR[1] = f0.y; dR[2] = f0.z; dR[3] = f0.w;
-        dR[4] = f1.x; dR[5] = f1.y; dR[6] = f1.z; dR[7] = f1.w;
-    } else {
-#pragma unroll
-        for (int jj = 0; jj < BJ; ++jj) { dT[jj] = 0.0f; dR[jj] = 0.0f; }
+        for (int j = 0; j < 4; ++j) {
+            dT.lo[j] = dhout[hb + (int64_t)(8 * q + j) * D + e];
+            dT.hi[j] = dhout[hb + (int64_t)(8 * q + 4 + j) * D + e];
+        }
+        dR.lo = *reinterpret_cast<const f32x4*>(dhout + hb + (int64_t)e * D + 8 * q);
+        dR.hi = *reinterpret_cast<const f32x4*>(dhout + hb + (int64_t)e * D + 8 * q + 4);
     }
 
+    // the state before a chunk, loaded a chunk ahead
+    auto load_state = [&](int c) __attribute__((always_inline)) {
+        const float* const src = c > 0 ? ckpt + hb * NC + (int64_t)(c - 1) * D * D : h_in ? h_in + hb : nullptr;
+        Rows8 S = zero;
+        if (src) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                S.lo[j] = (src + 8 * q * D)[j * D + e];
+                S.hi[j] = (src + 8 * q * D)[(4 + j) * D + e];
+            }
+        }
+        return S;
+    };
+    Rows8 Sst = load_state(NC - 1);
     stage_load(NC - 1);
     stage_store(NC - 1);
-    int u = 0;   // reverse step counter (parity of dsa_part, ring slot)
 
-    // Outputs of reverse step uu (time tt): 6 × 64 sums of 8 partials, 48 per
-    // wave so every wave carries the same share between two barriers.
-    const int fidx = q * (NOUT * D / BQ) + i;   // output index owned by this lane (i < 48)
+    // Outputs of the step in a ring slot: 6 × 64 sums of 8 partials, 48 per
+    // wave so every wave carries the same share between two barriers; the
+    // steps go out last to first, so the lane's address moves down by one.
+    const int fidx = q * (NOUT * D / BQ) + min(l, NOUT * D / BQ - 1);   // output index owned by this lane (l < 48)
     const int fo = fidx >> 6, fcol = fidx & 63;
-    auto flush = [&](int uu, int tt) {
-        if (i < NOUT * D / BQ)
-            store1<GT>(outs[fo], base0 + (int64_t)tt * strideT + fcol, sum8(&ring[uu % 3][fo][0][fcol]));
+    constexpr int64_t gsz = GT == RWKV_F32 ? 4 : 2;
+    char* fout = reinterpret_cast<char*>(fo == 0 ? g_dr : fo == 1 ? g_dw : fo == 2 ? g_dk : fo == 3 ? g_db : fo == 4 ? g_dv : g_da) +
+                 (base0 + (T - 1) * strideT + fcol) * gsz;
+    auto flush = [&](const Parts& p) __attribute__((always_inline)) {
+        if (l < NOUT * D / BQ) store1<GT>(fout, 0, p.sum());
+        fout -= strideT * gsz;
     };
+    auto flush_parts = [&](int slot) __attribute__((always_inline)) { return Parts(&ring[slot][fo][0][fcol]); };
 
     for (int c = NC - 1; c >= 0; --c) {
         __syncthreads();   // chunk c staged; every read of the other buffer is done
         if (c > 0) stage_load(c - 1);
-        float (*st)[CH][D] = stage[c & 1];
+        const float (*st)[CH][D] = stage[c & 1];
 
-        float Sst[BJ];     // state before the chunk
-        if (c > 0) {
-            const float* ck = ckpt + (hb * NC) + (int64_t)(c - 1) * D * D;
+        // the forward's state update: fma(w, S, fma(sa, b, v·k))
+        auto advance = [&](int s, const Rows8& S) __attribute__((always_inline)) {
+            const Rows8 n = outer8(st[7][s][e], st[5][s][e], outer8(st[3][s][e], st[2][s][e], zero));
+            const float wi = st[1][s][e];
+            return Rows8{S.lo * wi + n.lo, S.hi * wi + n.hi};
+        };
+        Rows8 h[CH + 1];   // h[s] = state before step s of the chunk
+        h[0] = Sst;
 #pragma unroll
-            for (int jj = 0; jj < BJ; ++jj) Sst[jj] = ck[(int64_t)(8 * q + jj) * D + i];
-        } else if (h_in) {
+        for (int s = 0; s < CH; ++s) h[s + 1] = advance(s, h[s]);
+        if (c > 0) Sst = load_state(c - 1);
+        float dr = dots8(st[6][CH - 1][jx], h[CH]).x0;   // the coming step's dr partial
 #pragma unroll
-            for (int jj = 0; jj < BJ; ++jj) Sst[jj] = h_in[hb + (int64_t)(8 * q + jj) * D + i];
-        } else {
-#pragma unroll
-            for (int jj = 0; jj < BJ; ++jj) Sst[jj] = 0.0f;
-        }
-
-#pragma unroll
-        for (int half = 1; half >= 0; --half) {
-            // states of the window: hist[m] = state before step WIN·half + m
-            float hist[WIN + 1][BJ];
-            float S0[BJ];
-#pragma unroll
-            for (int jj = 0; jj < BJ; ++jj) S0[jj] = Sst[jj];
-            if (half == 1) {
-#pragma unroll
-                for (int s = 0; s < WIN; ++s) {
-                    float N[BJ];
-                    bwd_recompute8(S0, N, st[3][s][jl], st[7][s][jl], st[2][s][i], st[5][s][i], st[1][s][i]);
-#pragma unroll
-                    for (int jj = 0; jj < BJ; ++jj) S0[jj] = N[jj];
-                }
-            }
-#pragma unroll
-            for (int jj = 0; jj < BJ; ++jj) hist[0][jj] = S0[jj];
-#pragma unroll
-            for (int m = 0; m < WIN; ++m) {
-                const int s = WIN * half + m;
-                bwd_recompute8(hist[m], hist[m + 1], st[3][s][jl], st[7][s][jl], st[2][s][i], st[5][s][i],
-                               st[1][s][i]);
-            }
-            // step vectors: own column i and broadcast row jl; the next step's
-            // are read before this step's barrier so they are ready after it
-            struct StepVec {
-                float ri, wi, ai, dyi, R, W, K, V, A, B, DY, SA;
-            };
-            auto load_vec = [&](int s) __attribute__((always_inline)) {
-                return StepVec{st[0][s][i], st[1][s][i], st[4][s][i], st[6][s][i], st[0][s][jl], st[1][s][jl],
-                               st[2][s][jl], st[3][s][jl], st[4][s][jl], st[5][s][jl], st[6][s][jl], st[7][s][jl]};
-            };
-            StepVec cur = load_vec(WIN * half + WIN - 1);
-#pragma unroll
-            for (int m = WIN - 1; m >= 0; --m, ++u) {
-                const int s = WIN * half + m;
-                const int t = c * CH + s;
-                const float (&Sa)[BJ] = hist[m + 1];
-                const float (&Sp)[BJ] = hist[m];
-                const float ri = cur.ri, wi = cur.wi, ai = cur.ai, dyi = cur.dyi;
-                const float R = cur.R, W = cur.W, K = cur.K, V = cur.V;
-                const float A = cur.A, B = cur.B, DY = cur.DY, SA = cur.SA;
-                float pdr = 0.0f, pdk = 0.0f, pdb = 0.0f, pdv = 0.0f, pds = 0.0f, pdw = 0.0f, pda = 0.0f;
-                RWKV_B1_BLOCK(0, 1, 2, 3, 0);
-                RWKV_B1_BLOCK(4, 5, 6, 7, 4);
-                {
-                    float w0 = 0.0f, w1 = 0.0f;
-#pragma unroll
-                    for (int jj = 0; jj < BJ; jj += 2) { w0 = fmaf(dT[jj], Sp[jj], w0); w1 = fmaf(dT[jj + 1], Sp[jj + 1], w1); }
-                    pdw = w0 + w1;
-                }
-                RWKV_B2_BLOCK(0, 1, 2, 3, 0);
-                RWKV_B2_BLOCK(4, 5, 6, 7, 4);
-                const int par = u & 1, slot = u % 3;
-                dsa_part[par][q][i] = pds;
-                ring[slot][0][q][i] = pdr;
-                ring[slot][1][q][i] = pdw;
-                ring[slot][2][q][i] = pdk;
-                ring[slot][3][q][i] = pdb;
-                ring[slot][4][q][i] = pdv;
-                StepVec nxt = cur;
-                if (m > 0) nxt = load_vec(s - 1);
-                __syncthreads();
-                const float dsa_i = sum8(&dsa_part[par][0][i]);
-                const float DS = __shfl(dsa_i, jl, 64);   // dsa of row 8q + (i & 7)
-                float nR[BJ], nT[BJ];
-                RWKV_B3_BLOCK(0, 1, 2, 3, 0);
-                RWKV_B3_BLOCK(4, 5, 6, 7, 4);
-#pragma unroll
-                for (int jj = 0; jj < BJ; ++jj) {
-                    dR[jj] = nR[jj];
-                    dT[jj] = fmaf(wi, dT[jj], nT[jj]);
-                }
-                ring[slot][5][q][i] = pda;
-                if (u > 0) flush(u - 1, t + 1);
-                cur = nxt;
-            }
+        for (int s = CH - 1; s >= 0; --s) {
+            const int par = s & 1, slot = s & 3;
+            const float re = st[0][s][e], we = st[1][s][e], ae = st[4][s][e], dye = st[6][s][e];
+            const float bk = st[odd ? 2 : 5][s][jx], vs = st[odd ? 7 : 3][s][jx], wj = st[1][s][jw];
+            // dS gains dy rᵀ; the wave's columns' share of dsa (and dv) and, from its rows, dk and db
+            dR = outer8(re, dye, dR);
+            dT = outer8(dye, re, dT);
+            __builtin_amdgcn_sched_barrier(0);
+            const Pair ds_dv = dots8(bk, dR);
+            const Pair kb = dots8(vs, dT);
+            __builtin_amdgcn_sched_barrier(0);
+            dsa_part[par][q][e] = ds_dv.x0;
+            const Rows8 tR = scale8(wj, dR);
+            const f32x4 pw = dT.lo * h[s].lo + dT.hi * h[s].hi;
+            ring[slot][0][q][e] = dr;
+            ring[slot][1][q][e] = (pw[0] + pw[1]) + (pw[2] + pw[3]);
+            ring[slot][2][q][e] = kb.x0;
+            ring[slot][3][q][e] = kb.x1;
+            ring[slot][4][q][e] = ds_dv.x1;
+            const Rows8 tT = {dT.lo * we, dT.hi * we};
+            const float dyx = st[6][s > 0 ? s - 1 : 0][jx];
+            __syncthreads();
+            const Parts pd(&dsa_part[par][0][e]), pf = flush_parts((s + 1) & 3);
+            const float dsa = pd.sum();
+            const float dsx = __shfl(dsa, (l >> 1) & 7, 64);
+            __builtin_amdgcn_sched_barrier(0);
+            dR = outer8(ae, dsa, tR);
+            dT = outer8(dsa, ae, tT);
+            const Pair ar = dots8(odd ? dyx : dsx, h[s]);
+            __builtin_amdgcn_sched_barrier(0);
+            ring[slot][5][q][e] = ar.x0;
+            dr = ar.x1;
+            if (s < CH - 1 || c < NC - 1) flush(pf);   // the step after this one's
         }
         if (c > 0) stage_store(c - 1);
     }
     __syncthreads();
-    flush(u - 1, 0);
-    float4* dst = reinterpret_cast<float4*>(dh_in + hb + (int64_t)i * D + 8 * q);
-    dst[0] = make_float4(dR[0], dR[1], dR[2], dR[3]);
-    dst[1] = make_float4(dR[4], dR[5], dR[6], dR[7]);
+    flush(flush_parts(0));
+    *reinterpret_cast<f32x4*>(dh_in + hb + (int64_t)e * D + 8 * q) = dR.lo;
+    *reinterpret_cast<f32x4*>(dh_in + hb + (int64_t)e * D + 8 * q + 4) = dR.hi;
 }
 
 // ─────────────────────────────── backward, row-owned (variant 1) ───────────────────────────────

@@ -28,8 +28,7 @@ wkv7_keep_forward_outputs = True
 _DT = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+_stream = _lib.stream
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

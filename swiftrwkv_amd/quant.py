@@ -404,20 +404,20 @@ def rwkvq_sym_interleave(codes_packed, qh, qh2, shape) -> np.ndarray:
 _OUT_DT = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+_stream = _lib.stream
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     """Contiguous with a 16-byte aligned base (the kernels use vector loads)."""
-    t = t.contiguous()
+    if not t.is_contiguous():
+        t = t.contiguous()
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def _dev_u8(t: torch.Tensor, numel: int, what: str) -> torch.Tensor:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError("quantised buffers must live on a ROCm device for the HIP kernels")
-    if t.dtype not in (torch.uint8, torch.int8):
+    if t.dtype is not torch.uint8 and t.dtype is not torch.int8:
         raise ValueError(f"{what}: expected a byte buffer, got {t.dtype}")
     if t.numel() != numel:
         raise ValueError(f"{what}: {t.numel()} bytes, the shape needs {numel}")
@@ -425,7 +425,7 @@ def _dev_u8(t: torch.Tensor, numel: int, what: str) -> torch.Tensor:
 
 
 def _dev_f16(t: torch.Tensor, numel: int, what: str) -> torch.Tensor:
-    if t.dtype != torch.float16:
+    if t.dtype is not torch.float16:
         raise ValueError(f"{what}: expected fp16 scales, got {t.dtype}")
     if t.numel() != numel:
         raise ValueError(f"{what}: {t.numel()} scales, the shape needs {numel}")
@@ -532,9 +532,9 @@ def rwkvq_sb6_gemv(x, qblk, qsqm, ddm, out_features: int, in_features: int, xbit
     if x.shape[0] % K:
         raise ValueError(f"sb6-GEMV: {x.shape[0]} input rows do not split over {K} fused matrices")
     N = x.shape[0] // K
-    x32 = _aligned(x.to(torch.float32))
+    x32 = _aligned(_lib.f32(x))
     qblk, qsqm, ddm = _sb6_bufs(qblk, qsqm, ddm, out_features, in_features, xbits)
-    y = torch.empty((N, out_features), dtype=torch.float32, device=x.device)
+    y = x32.new_empty((N, out_features))
     if out_per is None:
         _lib.call("rwkv_sb6_gemv", x32.data_ptr(), N, qblk.data_ptr(), qsqm.data_ptr(), ddm.data_ptr(),
                   y.data_ptr(), out_features, in_features, xbits, _stream(x32))
@@ -572,8 +572,8 @@ def _quant_gemm(entry: str, what: str, x, bufs, out_features: int, in_features: 
         x = x.unsqueeze(0)
     if x.dim() != 3 or x.shape[0] != G or x.shape[2] != in_features:
         raise ValueError(f"{what} GEMM: input {tuple(x.shape)}, expected [{G}, M, {in_features}]")
-    if x.dtype not in (torch.float32, torch.float16):
-        x = x.float()
+    if x.dtype is not torch.float16:
+        x = _lib.f32(x)
     x = _aligned(x)
     M = x.shape[1]
     ep = _GEMM_EP[epilogue]
@@ -716,7 +716,7 @@ def rwkvq_sb6_gemv_batch(x, qblk, qsqm, ddm, out_features: int, in_features: int
     if not rwkvq_sb6_gemv_batch_applies(N, out_features, in_features, xbits, per):
         raise ValueError(f"sb6 batched GEMV: N={N} [{out_features}, {in_features}] xbits={xbits} out_per={per} "
                          "not taken")
-    x32 = _aligned(x.to(torch.float32))
+    x32 = _aligned(_lib.f32(x))
     qblk, qsqm, ddm = _sb6_bufs(qblk, qsqm, ddm, out_features, in_features, xbits)
     ep = _GEMV_EP[epilogue]
     if out is None:
@@ -773,7 +773,7 @@ def rwkvq_sb6_gemv_batch_t16(x, tq, ts, tm, out_features: int, in_features: int,
     for t, n, dt in ((tq, nw // 2, torch.uint8), (ts, nw // 32, torch.float16), (tm, nw // 16, torch.bfloat16)):
         if not t.is_cuda or t.dtype != dt or not t.is_contiguous() or t.numel() != n:
             raise ValueError("sb6 batched GEMV: T16 buffers from rwkvq_sb6_t16 expected")
-    x32 = _aligned(x.to(torch.float32))
+    x32 = _aligned(_lib.f32(x))
     ep = _GEMV_EP[epilogue]
     if out is None:
         if ep == 1:
@@ -815,9 +815,9 @@ def rwkvq_sym_gemv(x, qblk, qs, d, out_features: int, in_features: int, bits: in
     if x.shape[0] % K:
         raise ValueError(f"sym-GEMV: {x.shape[0]} input rows do not split over {K} fused matrices")
     N = x.shape[0] // K
-    x32 = _aligned(x.to(torch.float32))
+    x32 = _aligned(_lib.f32(x))
     qblk, qs, d = _sym_bufs(qblk, qs, d, out_features, in_features, bits)
-    y = torch.empty((N, out_features), dtype=torch.float32, device=x.device)
+    y = x32.new_empty((N, out_features))
     _lib.call("rwkv_sym_gemv", x32.data_ptr(), N, qblk.data_ptr(), qs.data_ptr(), d.data_ptr(), y.data_ptr(),
               out_features, in_features, bits, per, _stream(x32))
     return y

@@ -246,6 +246,26 @@ def test_batched_fused_gemv_equals_separate_bitwise(orc):
         assert torch.equal(fused[:, i * OUT:(i + 1) * OUT], batch)
 
 
+# a fused batch stages a workgroup's own matrix only where its rows (up to
+# 8 waves x 64 / G) divide a matrix's: sizes on both sides of that line
+@pytest.mark.parametrize("OUT,IN", [(16, 2048), (32, 2048), (96, 2048), (32, 512), (64, 512), (192, 512)])
+def test_batched_fused_gemv_matrix_sizes_bitwise(orc, OUT, IN):
+    case(f"batched fused sym_8 / sb6 3x{OUT}x{IN}")
+    Kn, N = 3, 5
+    x = np.random.default_rng(OUT + IN).standard_normal((N * Kn, IN)).astype(np.float32)
+    for make, run in ((lambda i: sb6_tensor(orc, OUT, IN, 0, seed=60 + i),
+                       lambda z, w, o, per: Q.rwkvq_sb6_gemv(z, *w, o, IN, 0, out_per=per)),
+                      (lambda i: sym_tensor(orc, OUT, IN, 8, seed=60 + i),
+                       lambda z, w, o, per: Q.rwkvq_sym_gemv(z, *w, o, IN, 8, out_per=per))):
+        parts = [make(i) for i in range(Kn)]
+        w = [dev(np.concatenate([p[j] for p in parts])) for j in range(3)]
+        fused = run(dev(x), w, OUT * Kn, OUT)
+        for i, p in enumerate(parts):
+            for n in range(N):
+                alone = run(dev(x[n * Kn + i:n * Kn + i + 1]), [dev(z) for z in p], OUT, None)
+                assert torch.equal(fused[n:n + 1, i * OUT:(i + 1) * OUT], alone), (i, n)
+
+
 def test_gemv_is_deterministic(orc):
     case("gemv determinism")
     qblk, qsqm, ddm = sb6_tensor(orc, 3072, 768, 1, seed=3)

@@ -226,7 +226,7 @@ public final class RwkvqDeviceSidecar {
                                 inFeatures: info.inFeatures, bits: info.bits)
     }
 
-    /// The split-K workspace a long pass of M rows takes (nil: one K range).
+    /// The workspace a long pass of M rows takes (nil: one K range without).
     private func gemmWorkspace(_ M: Int, _ info: RwkvqTensorInfo) throws -> (DeviceArray?, Int64) {
         let n = rwkv_quant_gemm_workspace(Int64(M), Int64(info.outFeatures), Int64(info.inFeatures))
         return n > 0 ? (try DeviceArray(shape: [Int(n)], dtype: .uint8), n) : (nil, 0)

@@ -1044,8 +1044,7 @@ class RwkvqSidecar:
                 return y.to(x.dtype).reshape(*lead, OUT)
         if base_dtype == torch.float16:
             # the fp16 long pass on the matrix cores, from the packed bytes (the
-            # input rounded to fp16 here as the kernels would round it, so that
-            # shapes with many tiles can take the dense route)
+            # input rounded to fp16 here as the kernels would round it)
             xin = x2d.to(torch.float16)
             if info.kind == RwkvqKind.sb6 and rwkvq_sb6_gemm_applies(OUT, IN, info.xbits):
                 y = rwkvq_sb6_gemm(xin, self._buf(key, "qblk"), self._buf(key, "qsqm"), self._buf(key, "ddm"), OUT,

@@ -320,18 +320,27 @@ rwkv_status rwkv_sym_gemv_ep(const float* x, int64_t N,
  * workspace: NULL, or device memory of rwkv_quant_gemm_workspace(M, OUT, IN)
  * bytes (16-byte aligned; a smaller one is refused before any launch).  With
  * it, passes of few output tiles split the K sum over the waves of a workgroup
- * (a fixed order: deterministic, the same bound), and larger ones dequantise
- * the weight into the workspace (fp16, the dequant's values in the matrix
- * cores' order) and multiply from there — the same products in the same order
- * as one range, so bitwise its result.  Which one depends on the shape alone:
- * f32 inputs give the bits of f16 inputs of equal values.  With NULL the launch
- * is one range.  Launches sharing a workspace must not overlap. */
+ * or over ranges whose sums a second launch adds (a fixed order: deterministic,
+ * the same bound), and larger ones dequantise the weight into the workspace
+ * (fp16) and multiply from there — the same products in the same order as one
+ * range, so bitwise its result.  Which one depends on the shape and the format
+ * alone: f32 inputs give the bits of f16 inputs of equal values.  With NULL the
+ * launch is one range.  Launches sharing a workspace must not overlap. */
 int rwkv_sb6_gemm_applies(int64_t OUT, int64_t IN, int xbits, int64_t out_per);
 int64_t rwkv_quant_gemm_workspace(int64_t M, int64_t OUT, int64_t IN);
 rwkv_status rwkv_sb6_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda, int64_t x_group_stride,
                           const uint8_t* qblk, const uint8_t* qsqm, const uint16_t* ddm, void* y, int64_t ldy,
                           int64_t OUT, int64_t IN, int xbits, int64_t out_per, int epilogue, void* workspace,
                           int64_t workspace_bytes, void* stream);
+
+/* Which kernel rwkv_sb6_gemm (sym 0; bits = xbits) or rwkv_sym_gemm (sym 1)
+ * takes for a pass with contiguous rows (lda = IN) and this much workspace (< 0:
+ * NULL), as four ints: {0, tile rows, tile features, K ranges}, {1, tile rows,
+ * tile features (of f16 inputs), waves that split K}, {2, ...} a dequant in the
+ * matrix cores' order and a dense product, {3, ...} a row-major dequant and
+ * rwkv_f16_gemm's kernel.  Host only. */
+rwkv_status rwkv_quant_gemm_route(int sym, int bits, rwkv_dtype x_dt, int64_t M, int64_t OUT, int64_t IN,
+                                  int64_t out_per, int64_t workspace_bytes, int32_t* route);
 
 /* The same long pass for sym matrices (8-bit codes, or 6-bit in the loader's
  * interleave; qs [OUT, IN/16] int8, d [OUT, IN/256] fp16): fp16(W) is exactly

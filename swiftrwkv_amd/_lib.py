@@ -99,6 +99,7 @@ _SIGS = {
     "rwkv_sb6_gemm_applies": (I, [L, L, I, L]),
     "rwkv_sb6_gemm": (I, [P, I, L, L, L, P, P, P, P, L, L, L, I, L, I, P, L, P]),
     "rwkv_quant_gemm_workspace": (L, [L, L, L]),
+    "rwkv_quant_gemm_route": (I, [I, I, I, L, L, L, L, L, P]),
     "rwkv_f16_gemm_applies": (I, [L, L, L, L]),
     "rwkv_f16_gemm": (I, [P, L, L, L, P, P, L, L, L, L, I, P]),
     "rwkv_sym_gemm_applies": (I, [L, L, I, L]),

@@ -63,6 +63,8 @@ struct GemmArgs {
     void* y;              // [M][ldy]: fp32 (epilogues 0, 1) or fp16 (epilogue 2)
     int64_t ldy;
     int M, N, K, out_per;
+    float* part;          // splits > 1: the fp32 partial sums [splits][M][N]
+    int splits;           // K ranges quant_gemm_kernel divides a tile's stages into
 };
 
 // The epilogue of one output: fp16 rounding of the fp32 sum (the fp16
@@ -309,18 +311,17 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int gq = lane >> 4, li = lane & 15;
     // Workgroups are dealt to the 8 XCDs round-robin (id mod 8), each XCD with
-    // its own L2: XCD x takes the input row-blocks m ≡ x (mod 8) and sweeps
-    // every feature tile of one block before the next, so an input block is
-    // fetched into one L2 only.  The grid is padded to whole groups of 8 row
-    // blocks; a padding workgroup exits before any barrier.
-    const int ntn = g.N / BN;
-    const int total = ((g.M + BM - 1) / BM) * ntn;
+    // its own L2: XCD x takes a contiguous run of the (row block, feature
+    // block, K range) order, so an input block is read into one L2, or two.
+    const int ntn = g.N / BN, S = g.splits;
+    const int total = ((g.M + BM - 1) / BM) * ntn * S;
     const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
-    const int t = xcd * (total >> 3) + min(xcd, total & 7) + loc;   // the tile's place in (m, n) order
-    const int tile_n = t % ntn, tile_m = t / ntn;
+    const int t = xcd * (total >> 3) + min(xcd, total & 7) + loc;   // the tile's place in that order
+    const int kz = t % S, tile_n = (t / S) % ntn, tile_m = t / (S * ntn);
     const int n0 = tile_n * BN;
     const int m0 = tile_m * BM;
     const int nst = g.K / BK;
+    const int st0 = (int)((int64_t)kz * nst / S), st1 = (int)((int64_t)(kz + 1) * nst / S);
 
     // input rows of this tile come from the matrix group its output features belong to
     const TA* xg = reinterpret_cast<const TA*>(g.x) + (int64_t)(n0 / g.out_per) * g.x_gstride;
@@ -387,8 +388,8 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
         }
     };
 
-    auto ar = load_a(0);
-    BRaw bcur = load_b(0);
+    auto ar = load_a(st0);
+    BRaw bcur = load_b(st0);
     store_a(0, ar);
     half8 b0[NT], b1[NT];
     dequant(bcur, 0, b0);
@@ -397,9 +398,9 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
     // Per stage: the next stage's bytes are requested first; unit 0's
     // products run while unit 1 is decoded, unit 1's while the next stage's
     // unit 0 is (one MFMA, one VALU instruction, alternately).
-    for (int st = 0; st < nst; ++st) {
-        const int buf = st & 1;
-        const bool more = st + 1 < nst;
+    for (int st = st0; st < st1; ++st) {
+        const int buf = (st - st0) & 1;
+        const bool more = st + 1 < st1;
         BRaw bnxt = bcur;
         if (more) {
             ar = load_a(st + 1);
@@ -424,6 +425,19 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
         __syncthreads();
     }
 
+    if (S > 1) {   // this K range's fp32 sums; gemm_split_reduce adds the ranges and applies the epilogue
+        float* part = g.part + (int64_t)kz * g.M * g.N;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = m0 + 16 * i + 4 * gq + r;
+                if (row >= g.M) continue;
+#pragma unroll
+                for (int j = 0; j < NT; ++j) part[(int64_t)row * g.N + nb + 16 * j] = acc[i][j][r];
+            }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
 #pragma unroll
@@ -434,6 +448,28 @@ __global__ __launch_bounds__(256, 2) void quant_gemm_kernel(GemmArgs g) {
             for (int j = 0; j < NT; ++j) store_out<EP>(g.y, (int64_t)row * g.ldy + nb + 16 * j, acc[i][j][r]);
         }
     }
+}
+
+// The K ranges of a split launch summed in range order (a fixed order: the
+// result does not depend on which workgroup finished first), then the
+// epilogue of the one-range kernel: fp16 rounding, store / add / relu².
+// Thread i takes 4 consecutive outputs of one row (N is a multiple of 128).
+template <int EP>
+__global__ __launch_bounds__(256) void gemm_split_reduce(const float* __restrict__ part, int S, int M, int N,
+                                                         void* y, int64_t ldy) {
+    const int64_t n4 = (int64_t)M * N / 4;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const float4* p = reinterpret_cast<const float4*>(part) + i;
+    float4 a = p[0];
+    for (int k = 1; k < S; ++k) {
+        const float4 b = p[(int64_t)k * n4];
+        a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+    }
+    const int64_t row = 4 * i / N, col = 4 * i % N;
+    const float v[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) store_out<EP>(y, row * ldy + col + c, v[c]);
 }
 
 // ── few output tiles: the K sum split over the waves of a workgroup ──
@@ -471,14 +507,9 @@ struct KsArgs {
 
 // LDS bytes per staged weight row: the four units' bytes in an odd number of
 // 16-byte chunks, so 16 rows' reads at one column fall on distinct banks.
-template <class F>
-constexpr int ks_brow() {
-    constexpr int chunks = 4 * F::UB / 16;
-    return 16 * (chunks | 1);
-}
-template <class F>
-constexpr int ks_wave_lds(int mt, int nt) {
-    return 16 * mt * KS_AROW + 16 * nt * (ks_brow<F>() + ks_srow(nt));
+constexpr int ks_brow(int unit_bytes) { return 16 * ((4 * unit_bytes / 16) | 1); }
+constexpr int ks_wave_lds(int unit_bytes, int mt, int nt) {
+    return 16 * mt * KS_AROW + 16 * nt * (ks_brow(unit_bytes) + ks_srow(nt));
 }
 
 template <class F, typename TA, int MT, int NT, int MAXW>
@@ -502,9 +533,9 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_ks_kernel(KsArgs ka) {
     const int steps = g.K / KS_COLS, NU = g.K >> 5;
     const int p0 = wave * steps / W, p1 = (wave + 1) * steps / W;   // W <= steps: at least one step each
 
-    unsigned char* const mine = lds + wave * ks_wave_lds<F>(MT, NT);
+    unsigned char* const mine = lds + wave * ks_wave_lds(F::UB, MT, NT);
     unsigned char* const mb = mine + BM * KS_AROW;
-    unsigned char* const ms = mb + BN * ks_brow<F>();
+    unsigned char* const ms = mb + BN * ks_brow(F::UB);
 
     // Uniform bases (tile, step) plus a 32-bit offset per load.
     const char* xt = reinterpret_cast<const char*>(reinterpret_cast<const TA*>(g.x) +
@@ -534,7 +565,7 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_ks_kernel(KsArgs ka) {
 #pragma unroll
         for (int e = 0; e < BL; ++e) {
             const int id = min(lane + 64 * e, BN * BC - 1);
-            *reinterpret_cast<u32x4*>(mb + id / BC * ks_brow<F>() + id % BC * 16) = rb[e];
+            *reinterpret_cast<u32x4*>(mb + id / BC * ks_brow(F::UB) + id % BC * 16) = rb[e];
         }
 #pragma unroll
         for (int e = 0; e < AL; ++e) {
@@ -593,7 +624,7 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_ks_kernel(KsArgs ka) {
         for (int h = 0; h < 2; ++h) {
             typename F::Codes cd[NT];
 #pragma unroll
-            for (int j = 0; j < NT; ++j) cd[j] = F::load_codes(mb + (16 * j + li) * ks_brow<F>() + 2 * h * F::UB, gq);
+            for (int j = 0; j < NT; ++j) cd[j] = F::load_codes(mb + (16 * j + li) * ks_brow(F::UB) + 2 * h * F::UB, gq);
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 half8 b[NT];
@@ -872,7 +903,8 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN > 4 ? 1 : 2) void dense_tiles
 // ── dense fp16 weights, row-major ──
 //
 // y = epilogue(fp16(x · wᵀ)) for x [groups][M][lda] fp16 and w [N][K] fp16
-// (rows K-contiguous): a dense fp16 base (rwkv_f16_gemm).
+// (rows K-contiguous): a dense fp16 base (rwkv_f16_gemm), and quantised passes
+// of many rows and a short K (gemm_route).
 //
 // A workgroup of 8 waves computes a 256 (input rows) × 256 (output features)
 // tile in stages of 64 columns.  Both operands are staged in LDS as rows of
@@ -1038,6 +1070,53 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(DenseArgs g) {
     }
 }
 
+// Which kernel a quantised pass takes when the caller gave a workspace, by
+// shape and weight format alone: fp32 inputs take the same sums as fp16 ones
+// (an input is rounded to fp16 either way, so equal values give equal results).
+// Times in µs, fitted on MI355X to graph-timed calls of every kernel at 11,000
+// points (1-16,400 rows, 256-26,900 × 256-14,800 matrices, all five formats;
+// the pick is within 15 % of the fastest kernel at 95 of 100 fp16 points).  In
+// x rounds of the 256 CUs:
+//   * Waves splitting K (gemm_ks_kernel): workgroups of W waves share a CU as
+//     LDS and registers allow (occ); a round of occ costs a start plus its K,
+//     longer by rho for each workgroup more.  A wave's steps are whole, so K
+//     counts half as it is and half rounded up to W waves.  Against one launch
+//     with K ranges and their reduction: 128 rows × 3072 × 768 6.5 (13.1), 128
+//     × 768 × 3072 7.0 (16.1), 16 × 4096 × 4096 7.6 (22.8).  Its weights are
+//     decoded once per row block, so many row blocks favour:
+//   * the dense route (dequant_tiles_kernel + dense_tiles_kernel): the dequant
+//     (a launch plus its bytes), the output's bytes, then per 64-column stage
+//     the latency of one tile or the rate of a full CU.  Against the same: 1001
+//     × 3072 × 1024 21.7 (32.9), 4096 × 1024 × 4096 44.7 (134).
+//   * the dense route over row-major weights (rwkv_*_dequant +
+//     dense_gemm_kernel; fp16 inputs): one round costs more, but each tile
+//     starts and ends sooner, which tells up to K ~ 1024: 8192 × 3072 × 256
+//     31.9 (37.5 over operand order), 4177 × 12288 × 768 107 (117), 8192 ×
+//     4096 × 1024 77 (78), 4096 × 4096 × 4096 126 (119).
+//   * K ranges on 128 × 128 tiles (quant_gemm_kernel), where a tile's 128 rows
+//     save a decode: 65-128 rows of 3584 features or more (98 × 10240 × 5888
+//     sb6 4-bit 45 (52 split over waves), 128 × 14336 × 14336 sym 8-bit 148
+//     (224); fewer features split over waves are faster throughout), and one
+//     range, without a dequant, up to K = 1024 (512 × 12288 × 256 14.8 (18.5)).
+struct GemmRoute {
+    enum Kind { kRanges, kSplitWaves, kDense, kDenseRows } kind = kRanges;
+    int tm = 128, tn = 128;   // the tile (kSplitWaves: with fp16 inputs; kDenseRows: that of kDense, for fp32 inputs)
+    int parts = 1;            // what K is split over: ranges or waves
+};
+
+// Weight formats: sb6 by xbits, then sym 8- and 6-bit.
+enum GemmFormat { kSb6 = 0, kSym8 = 3, kSym6 = 4, kFormats = 5 };
+
+// K ranges of a launch on 128 × 128 tiles: one where the (row block, feature
+// block) tiles already fill the chip; otherwise enough to reach about 384
+// workgroups (two per CU hold 512), each range at least 3 stages of 64 columns.
+int gemm_splits(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((M + 127) / 128) * (N / 128);
+    if (tiles >= 160) return 1;
+    const int64_t want = (384 + tiles - 1) / tiles, most = K / BK / 3;
+    return (int)std::max<int64_t>(1, std::min(want, most));
+}
+
 // The dense kernel's shapes (x rows lda halves apart, group g at x + g·x_gstride).
 bool dense_shape_ok(int64_t M, int64_t OUT, int64_t IN, int64_t out_per, int64_t lda) {
     return M >= 1 && M <= ((int64_t)1 << 24) && OUT >= DT && OUT % DT == 0 && OUT <= ((int64_t)1 << 30) &&
@@ -1046,80 +1125,112 @@ bool dense_shape_ok(int64_t M, int64_t OUT, int64_t IN, int64_t out_per, int64_t
            ((M + DT - 1) / DT) * (OUT / DT) < ((int64_t)1 << 31);
 }
 
-// Which kernel a quantised pass takes when the caller gave a workspace, by
-// shape alone: fp32 inputs take the same sums as fp16 ones (an input is
-// rounded to fp16 either way, so equal values give equal results).  Times in
-// µs, fitted to graph-timed calls on MI355X (sb6 4-bit, 4-4096 rows, 768-8192 ×
-// 768-4096 matrices; within ~20 %): a workgroup's time is a start plus its K,
-// and CUs take ceil(workgroups / 256) of them in turn.
-//   * Waves splitting K (gemm_ks_kernel): A + B·K/1024 per tile.  Against one
-//     fused launch with K ranges and their reduction: 128 rows × 3072 × 768
-//     6.5 (13.1), 128 × 768 × 3072 7.0 (16.1), 16 × 4096 × 4096 7.6 (22.8),
-//     512 × 1024 × 4096 18.2 (28.3).  Its weights are decoded once per row
-//     block, so many row blocks favour:
-//   * the dense route (dequant_tiles_kernel + dense_tiles_kernel): the dequant
-//     (a launch plus its bytes), then per 64-column stage the latency of one
-//     tile or the rate of a full CU.  Against the same: 1001 × 3072 × 1024
-//     21.7 (32.9), 2048 × 1024 × 4096 30.2 (61), 4096 × 1024 × 4096 44.7 (134);
-//     against a row-major weight through LDS 4096 × 4096 × 4096 119 (126).
-struct GemmRoute {
-    enum Kind { kFused, kSplitWaves, kDense } kind = kFused;
-    int mt = 0, nt = 0;   // kSplitWaves: the tile / 16 (fp16 inputs)
-    int waves = 0;
-    int tile = 0;         // kDense: the tile shape's id
-};
+// Bytes of workspace a route uses.
+int64_t route_bytes(const GemmRoute& r, int64_t M, int64_t N, int64_t K) {
+    if (r.kind == GemmRoute::kDense || r.kind == GemmRoute::kDenseRows) return N * K * 2;   // the fp16 weight
+    return r.kind == GemmRoute::kRanges && r.parts > 1 ? r.parts * M * N * 4 : 0;
+}
 
-GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, int64_t out_per, int64_t lda) {
-    const auto blocks = [&](int tm, int tn) { return (double)((M + tm - 1) / tm) * (double)(N / tn); };
-    const double k = (double)K / 1024, st = (double)K / DKS;
+// The fastest route within `bytes` of workspace.
+GemmRoute gemm_route(int fmt, int64_t M, int64_t N, int64_t K, int64_t out_per, int64_t lda, int64_t bytes) {
+    const double steps = (double)K / KS_COLS, st = (double)K / DKS;
+    const double nk = (double)N * (double)K / 1e6, mn = (double)M * (double)N / 1e6;
+    const auto rounds = [&](int tm, int tn) { return (double)((M + tm - 1) / tm) * (double)(N / tn) / 256; };
     GemmRoute best;
     double cost = 1e30;
+    const auto offer = [&](double c, const GemmRoute& r) {
+        if (c >= cost || route_bytes(r, M, N, K) > bytes) return;
+        cost = c;
+        best = r;
+    };
+
+    static const int unit_bytes[kFormats] = {Sb6W<0>::UB, Sb6W<1>::UB, Sb6W<2>::UB, SymW<8>::UB, SymW<6>::UB};
     struct Ks {
         int mt, nt, waves, many;   // waves per workgroup: one round of the CUs, more
-        double a, b;
+        double a, rho, b[kFormats];
     };
-    static const Ks ks[] = {{1, 1, 8, 8, 3.0, 0.95},  {2, 1, 12, 6, 3.3, 1.07}, {2, 2, 8, 8, 3.5, 1.8},
-                            {4, 1, 8, 4, 3.6, 1.75}, {4, 2, 7, 7, 3.9, 2.9},   {4, 4, 6, 6, 3.0, 6.8}};
+    static const Ks ks[] = {{1, 1, 8, 8, 1.17, 1.00, {0.77, 0.96, 1.09, 0.89, 1.13}},
+                            {2, 1, 12, 6, 1.19, 1.18, {1.00, 1.18, 1.29, 1.11, 1.40}},
+                            {2, 2, 8, 8, 1.66, 0.94, {1.54, 1.93, 2.06, 1.66, 2.13}},
+                            {4, 1, 8, 4, 1.62, 1.21, {1.33, 1.47, 1.59, 1.69, 1.60}},
+                            {4, 2, 7, 7, 2.19, 1.42, {2.50, 2.88, 3.37, 2.88, 3.41}},
+                            {4, 4, 6, 6, 2.10, 1.40, {5.12, 6.02, 7.66, 7.15, 7.65}}};
     for (const Ks& e : ks) {
         // offsets within a tile's input rows are 32-bit
         if ((int64_t)16 * e.mt * lda * 4 >= ((int64_t)1 << 31)) continue;
-        const double n = std::ceil(blocks(16 * e.mt, 16 * e.nt) / 256);
-        // 64 × 16 tiles of four waves share a CU past one round
-        const double c = 2 + n * (e.mt == 4 && e.nt == 1 && n > 1 ? 1.1 + 1.6 * k : e.a - 2 + e.b * k);
-        if (c >= cost) continue;
-        cost = c;
-        int w = n > 1 ? e.many : e.waves;
+        const double x = rounds(16 * e.mt, 16 * e.nt);
+        const int lds = ks_wave_lds(unit_bytes[fmt], e.mt, e.nt);
+        int w = x > 1 ? e.many : e.waves;
         if (e.mt * e.nt == 1 && K >= 4096) w = 16;
-        w = (int)std::min<int64_t>(w, K / KS_COLS);
-        best = {GemmRoute::kSplitWaves, e.mt, e.nt, w, 0};
+        w = (int)std::min<int64_t>({(int64_t)w, K / KS_COLS, (int64_t)(KS_LDS / lds)});
+        // 16 waves of up to 128 registers
+        const int occ = std::max(1, std::min({(int)(KS_LDS / (w * lds)), 16 / w, 4}));
+        const double kb = e.b[fmt] * (steps + std::ceil(steps / w) * w) / 16;
+        const double whole = std::floor(x / occ), part = x - whole * occ;
+        offer(2 + whole * (e.a + kb * (1 + e.rho * (occ - 1))) +
+                  (part > 0 ? e.a + kb * (1 + e.rho * (std::ceil(part) - 1)) : 0.0),
+              {GemmRoute::kSplitWaves, 16 * e.mt, 16 * e.nt, w});
     }
+
     struct Tile {
-        int tm, tn, id;
-        double latency, rate;   // per stage: one tile alone, a tile on a full chip
+        int tm, tn;
+        double start, dequant, out;   // dequant, out: per 10^6 weights, outputs
+        double big;                   // per 10^6 weights past what the MALL holds of them
+        double latency, rate;         // per stage: one tile alone, a tile on a full chip
     };
-    static const Tile tiles[] = {
-        {64, 64, 64, 0.265, 0.21}, {64, 128, 128, 0.34, 0.34}, {128, 128, 256, 0.465, 0.52}, {256, 256, 512, 1.2, 1.7}};
+    const auto dense = [&](const Tile& t) {
+        const double n = rounds(t.tm, t.tn), whole = std::floor(n), part = n - whole;
+        return t.start + t.dequant * nk + t.big * std::max(0.0, nk - 128) + t.out * mn +
+               st * (whole * t.rate + (part > 0 ? std::max(t.latency, t.rate * part) : 0.0));
+    };
+    static const Tile tiles[] = {{64, 64, 6.95, 0.62, 1.20, 1.00, 0.182, 0.185},
+                                 {64, 128, 6.92, 0.66, 0.78, 1.03, 0.258, 0.314},
+                                 {128, 128, 8.45, 0.60, 0.74, 0.72, 0.386, 0.434},
+                                 {256, 256, 12.2, 0.64, 0.88, 0.62, 0.976, 1.35}};
+    static const Tile row_major = {256, 256, 7.87, 0.62, 0.73, 0.50, 0.923, 1.46};
+    const Tile* tile = nullptr;   // the fastest operand-ordered one
+    double tile_cost = 1e30;
     for (const Tile& t : tiles) {
         if (N % t.tn || out_per % t.tn || (int64_t)t.tm * lda * 4 >= ((int64_t)1 << 31) ||
             (int64_t)t.tn * K * 2 >= ((int64_t)1 << 31))
             continue;
-        const double n = blocks(t.tm, t.tn) / 256, whole = std::floor(n), part = n - whole;
-        const double per_stage = whole * t.rate + (part > 0 ? std::max(t.latency, t.rate * part) : 0.0);
-        const double c = 5.7 + (double)N * (double)K / 2.4e6 + st * per_stage;
-        if (c >= cost) continue;
-        cost = c;
-        best = {GemmRoute::kDense, 0, 0, 0, t.id};
+        const double c = dense(t);
+        if (c >= tile_cost) continue;
+        tile_cost = c;
+        tile = &t;
+    }
+    if (tile) offer(tile_cost, {GemmRoute::kDense, tile->tm, tile->tn, 1});
+    // the row-major dequant's thread index is 32-bit
+    if (tile && dense_shape_ok(M, N, K, out_per, lda) && N * (K / 8) < INT32_MAX)
+        offer(dense(row_major), {GemmRoute::kDenseRows, tile->tm, tile->tn, 1});
+
+    const int64_t blocks = ((M + 127) / 128) * (N / 128);
+    const int S = gemm_splits(M, N, K);
+    if (S == 1 ? blocks >= 160 && K <= 1024 : M > 64 && M <= 128 && blocks >= 28) {
+        static const double per_stage[kFormats] = {1.67, 2.24, 2.25, 1.66, 2.18};
+        const double x = rounds(128, 128) * S, whole = std::floor(x / 2), part = x - 2 * whole;
+        const double pitch = K % 2048 == 0 ? 1.21 : K % 1024 == 0 ? 1.09 : 1.0;   // its lanes are rows apart
+        // a tie goes to the ranges
+        offer((2.1 + (S > 1 ? 3.65 + 1.27 * S * mn : 0.45 * mn) +
+               pitch * per_stage[fmt] * st / S *
+                   (whole * 1.34 + (part > 0 ? 1 + 0.34 * std::max(0.0, part - 1) : 0.0))) *
+                  (S > 1 ? 0.97 : 1.0),
+              {GemmRoute::kRanges, 128, 128, S});
     }
     return best;
 }
 
-// Bytes of workspace a pass of this shape takes: the dense route's fp16 weight.
-// The split over waves needs none of its own; it asks for two ranges' fp32
-// sums, the least that a caller's workspace for such a shape has held, so that
-// the size still tells which shapes want one.
+// Bytes of workspace a pass of this shape takes, whatever the format.  The
+// split over waves needs none of its own; it asks for two ranges' fp32 sums,
+// the least that a caller's workspace for such a shape has held, so that the
+// size still tells which shapes want one.
 int64_t gemm_workspace(int64_t M, int64_t N, int64_t K) {
-    const GemmRoute r = gemm_route(M, N, K, N, K);
-    return r.kind == GemmRoute::kDense ? N * K * 2 : r.kind == GemmRoute::kSplitWaves ? 2 * M * N * 4 : 0;
+    int64_t need = 0;
+    for (int f = 0; f < kFormats; ++f) {
+        const GemmRoute r = gemm_route(f, M, N, K, N, K, INT64_MAX);
+        need = std::max(need, r.kind == GemmRoute::kSplitWaves ? 2 * M * N * 4 : route_bytes(r, M, N, K));
+    }
+    return need;
 }
 
 template <int EP>
@@ -1141,8 +1252,13 @@ void launch_dense(const DenseArgs& g, int epilogue, hipStream_t s) {
 // not hidden).
 template <class F, typename TA, int EP>
 void launch_gemm(const GemmArgs& g, hipStream_t s) {
-    const int64_t blocks = (int64_t)((g.M + 127) / 128) * (g.N / 128);
+    const int64_t blocks = (int64_t)((g.M + 127) / 128) * (g.N / 128) * g.splits;
     rwkv::launch(quant_gemm_kernel<F, TA, EP, 8, 2>, dim3((unsigned)blocks), dim3(256), s, g);
+    if (g.splits > 1) {
+        const int64_t n4 = (int64_t)g.M * g.N / 4;
+        rwkv::launch(gemm_split_reduce<EP>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), s, g.part, g.splits,
+                     g.M, g.N, g.y, g.ldy);
+    }
 }
 
 // y rows take aligned 4-wide accesses.
@@ -1154,7 +1270,7 @@ template <class F, typename TA, int MT, int NT, int MAXW>
 void launch_ks_tile(const KsArgs& a, int W, hipStream_t s) {
     constexpr int BM = 16 * MT, BN = 16 * NT;
     const int64_t blocks = (int64_t)((a.g.M + BM - 1) / BM) * (a.g.N / BN);
-    const size_t lds = (size_t)W * std::max(BM * (BN + KS_PAD) * 4, ks_wave_lds<F>(MT, NT));
+    const size_t lds = (size_t)W * std::max(BM * (BN + KS_PAD) * 4, ks_wave_lds(F::UB, MT, NT));
     rwkv::launch_lds(gemm_ks_kernel<F, TA, MT, NT, MAXW>, dim3((unsigned)blocks), dim3(64 * W), lds, s, a);
 }
 
@@ -1163,8 +1279,7 @@ void launch_ks_tile(const KsArgs& a, int W, hipStream_t s) {
 template <class F, typename TA>
 void launch_ks(const GemmArgs& g, const GemmRoute& r, int epilogue, hipStream_t s) {
     const KsArgs a{g, epilogue, vec_rows(g, epilogue)};
-    const int t = 10 * r.mt + r.nt;
-    const int W = std::min<int>(r.waves, (int)(KS_LDS / ks_wave_lds<F>(r.mt, r.nt)));
+    const int t = 10 * (r.tm / 16) + r.tn / 16, W = r.parts;
     if (t == 11) launch_ks_tile<F, TA, 1, 1, 16>(a, W, s);
     else if (t == 21) launch_ks_tile<F, TA, 2, 1, 12>(a, W, s);
     else if (t == 22) launch_ks_tile<F, TA, 2, 2, 8>(a, W, s);
@@ -1186,30 +1301,30 @@ void launch_tiles_shape(const DenseTArgs& g, hipStream_t s) {
 }
 
 template <typename TA, int EP>
-void launch_tiles_ep(const DenseTArgs& g, int tile, hipStream_t s) {
-    switch (tile) {
-        case 64: launch_tiles_shape<TA, EP, 1, 4, 4, 1, 4, 4>(g, s); break;     // 64 × 64
-        case 128: launch_tiles_shape<TA, EP, 1, 4, 4, 2, 4, 2>(g, s); break;    // 64 × 128
-        case 256: launch_tiles_shape<TA, EP, 1, 4, 8, 2, 4, sizeof(TA) == 2 ? 2 : 1>(g, s); break;    // 128 × 128
+void launch_tiles_ep(const DenseTArgs& g, const GemmRoute& r, hipStream_t s) {
+    switch (r.tm * r.tn) {
+        case 64 * 64: launch_tiles_shape<TA, EP, 1, 4, 4, 1, 4, 4>(g, s); break;
+        case 64 * 128: launch_tiles_shape<TA, EP, 1, 4, 4, 2, 4, 2>(g, s); break;
+        case 128 * 128: launch_tiles_shape<TA, EP, 1, 4, 8, 2, 4, sizeof(TA) == 2 ? 2 : 1>(g, s); break;
         default: launch_tiles_shape<TA, EP, 2, 4, 8, 4, 2, 1>(g, s); break;     // 256 × 256
     }
 }
 
 template <typename TA>
-void launch_tiles_ta(const DenseTArgs& a, int tile, int epilogue, hipStream_t s) {
-    if (epilogue == 0) launch_tiles_ep<TA, 0>(a, tile, s);
-    else if (epilogue == 1) launch_tiles_ep<TA, 1>(a, tile, s);
-    else launch_tiles_ep<TA, 2>(a, tile, s);
+void launch_tiles_ta(const DenseTArgs& a, const GemmRoute& r, int epilogue, hipStream_t s) {
+    if (epilogue == 0) launch_tiles_ep<TA, 0>(a, r, s);
+    else if (epilogue == 1) launch_tiles_ep<TA, 1>(a, r, s);
+    else launch_tiles_ep<TA, 2>(a, r, s);
 }
 
 // The dense route: dequantise into the workspace (operand order), then multiply.
 template <class F>
-void launch_tiles(const GemmArgs& g, int tile, bool f16, void* workspace, int epilogue, hipStream_t s) {
+void launch_tiles(const GemmArgs& g, const GemmRoute& r, bool f16, void* workspace, int epilogue, hipStream_t s) {
     _Float16* w = reinterpret_cast<_Float16*>(workspace);
     const int64_t waves = (int64_t)(g.N / 16) * (g.K / 128);
     rwkv::launch(dequant_tiles_kernel<F>, dim3((unsigned)((waves + 3) / 4)), dim3(256), s, g, w);
     const DenseTArgs a{g.x, g.lda, g.x_gstride, w, g.y, g.ldy, g.M, g.N, g.K, g.out_per, vec_rows(g, epilogue)};
-    f16 ? launch_tiles_ta<_Float16>(a, tile, epilogue, s) : launch_tiles_ta<float>(a, tile, epilogue, s);
+    f16 ? launch_tiles_ta<_Float16>(a, r, epilogue, s) : launch_tiles_ta<float>(a, r, epilogue, s);
 }
 
 template <class F>
@@ -1221,12 +1336,25 @@ void launch_gemm_ep(const GemmArgs& g, bool f16, int epilogue, hipStream_t s) {
     }
 }
 
+// Any kind but kDenseRows.
 template <class F>
-void launch_routed(const GemmArgs& g, const GemmRoute& r, bool f16, void* workspace, int epilogue, hipStream_t s) {
-    if (r.kind == GemmRoute::kDense) launch_tiles<F>(g, r.tile, f16, workspace, epilogue, s);
-    else if (r.kind == GemmRoute::kSplitWaves)
+void launch_routed(GemmArgs g, const GemmRoute& r, bool f16, void* workspace, int epilogue, hipStream_t s) {
+    if (r.kind == GemmRoute::kDense) {
+        launch_tiles<F>(g, r, f16, workspace, epilogue, s);
+    } else if (r.kind == GemmRoute::kSplitWaves) {
         f16 ? launch_ks<F, _Float16>(g, r, epilogue, s) : launch_ks<F, float>(g, r, epilogue, s);
-    else launch_gemm_ep<F>(g, f16, epilogue, s);
+    } else {
+        g.part = reinterpret_cast<float*>(workspace);
+        g.splits = r.parts;
+        launch_gemm_ep<F>(g, f16, epilogue, s);
+    }
+}
+
+// The dense route over row-major weights, once the workspace holds them.
+void launch_rows(const GemmArgs& g, const void* workspace, int epilogue, hipStream_t s) {
+    launch_dense(DenseArgs{reinterpret_cast<const _Float16*>(g.x), g.lda, g.x_gstride,
+                           reinterpret_cast<const _Float16*>(workspace), g.y, g.ldy, g.M, g.N, g.K, g.out_per},
+                 epilogue, s);
 }
 
 bool gemm_shape_ok(int64_t OUT, int64_t IN, int64_t out_per) {
@@ -1266,9 +1394,37 @@ rwkv_status gemm_workspace_check(const char* who, int64_t M, int64_t N, int64_t 
     return RWKV_OK;
 }
 
+// The route of an entry's call: one K range without a workspace.
+GemmRoute entry_route(int fmt, rwkv_dtype x_dt, int64_t M, int64_t N, int64_t K, int64_t out_per, int64_t lda,
+                      const void* workspace, int64_t workspace_bytes) {
+    GemmRoute r;
+    if (workspace) r = gemm_route(fmt, M, N, K, out_per, lda, workspace_bytes);
+    // row-major weights meet fp16 inputs only; operand order gives the same bits
+    if (r.kind == GemmRoute::kDenseRows && x_dt != RWKV_F16) r.kind = GemmRoute::kDense;
+    return r;
+}
+
 }  // namespace
 
 extern "C" {
+
+rwkv_status rwkv_quant_gemm_route(int sym, int bits, rwkv_dtype x_dt, int64_t M, int64_t OUT, int64_t IN,
+                                  int64_t out_per, int64_t workspace_bytes, int32_t* route) {
+    RWKV_REQUIRE(route, RWKV_E_NULL, "quant_gemm_route: null output");
+    RWKV_REQUIRE(sym ? rwkv_sym_gemm_applies(OUT, IN, bits, out_per) : rwkv_sb6_gemm_applies(OUT, IN, bits, out_per),
+                 RWKV_E_UNSUPPORTED, "quant_gemm_route: [%lld, %lld] bits %d out_per %lld not taken", (long long)OUT,
+                 (long long)IN, bits, (long long)out_per);
+    RWKV_REQUIRE(M >= 1 && M <= ((int64_t)1 << 24), RWKV_E_SHAPE, "quant_gemm_route: M (%lld) out of range", (long long)M);
+    RWKV_REQUIRE(x_dt == RWKV_F32 || x_dt == RWKV_F16, RWKV_E_DTYPE, "quant_gemm_route: inputs are f32 or f16");
+    const GemmRoute r = entry_route(sym ? (bits == 8 ? kSym8 : kSym6) : kSb6 + bits, x_dt, M, OUT, IN, out_per, IN,
+                                    workspace_bytes < 0 ? nullptr : route, workspace_bytes);
+    route[0] = r.kind;
+    route[1] = r.kind == GemmRoute::kDenseRows ? DT : r.tm;
+    route[2] = r.kind == GemmRoute::kDenseRows ? DT : r.tn;
+    route[3] = r.parts;
+    rwkv::clear_error();
+    return RWKV_OK;
+}
 
 int64_t rwkv_quant_gemm_workspace(int64_t M, int64_t OUT, int64_t IN) {
     if (M < 1 || M > ((int64_t)1 << 24) || OUT < 128 || OUT % 128 != 0 || IN < 256 || IN % 256 != 0) return 0;
@@ -1292,12 +1448,15 @@ rwkv_status rwkv_sb6_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda
     c = gemm_workspace_check("sb6_gemm", M, OUT, IN, workspace, workspace_bytes);
     if (c != RWKV_OK) return c;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    GemmArgs g{x, lda, x_group_stride, qblk, qsqm, ddm, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per};
+    const GemmArgs g{x, lda, x_group_stride, qblk, qsqm, ddm, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per, nullptr, 1};
     const bool f16 = x_dt == RWKV_F16;
-    // one K range without a workspace
-    const GemmRoute r = workspace ? gemm_route(M, OUT, IN, out_per, lda) : GemmRoute{};
+    const GemmRoute r = entry_route(kSb6 + xbits, x_dt, M, OUT, IN, out_per, lda, workspace, workspace_bytes);
     if (r.kind == GemmRoute::kDense) rwkv::counters().sb6_dequant.fetch_add(1);
-    if (xbits == 0) launch_routed<Sb6W<0>>(g, r, f16, workspace, epilogue, s);
+    if (r.kind == GemmRoute::kDenseRows) {
+        c = rwkv_sb6_dequant(qblk, qsqm, ddm, workspace, RWKV_F16, OUT, IN, xbits, stream);
+        if (c != RWKV_OK) return c;
+        launch_rows(g, workspace, epilogue, s);
+    } else if (xbits == 0) launch_routed<Sb6W<0>>(g, r, f16, workspace, epilogue, s);
     else if (xbits == 1) launch_routed<Sb6W<1>>(g, r, f16, workspace, epilogue, s);
     else launch_routed<Sb6W<2>>(g, r, f16, workspace, epilogue, s);
     RWKV_REQUIRE(hipGetLastError() == hipSuccess, RWKV_E_HIP, "sb6_gemm: launch failed");
@@ -1323,12 +1482,15 @@ rwkv_status rwkv_sym_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda
     c = gemm_workspace_check("sym_gemm", M, OUT, IN, workspace, workspace_bytes);
     if (c != RWKV_OK) return c;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    GemmArgs g{x, lda, x_group_stride, qblk, qs, d, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per};
+    const GemmArgs g{x, lda, x_group_stride, qblk, qs, d, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per, nullptr, 1};
     const bool f16 = x_dt == RWKV_F16;
-    // one K range without a workspace
-    const GemmRoute r = workspace ? gemm_route(M, OUT, IN, out_per, lda) : GemmRoute{};
+    const GemmRoute r = entry_route(bits == 8 ? kSym8 : kSym6, x_dt, M, OUT, IN, out_per, lda, workspace, workspace_bytes);
     if (r.kind == GemmRoute::kDense) rwkv::counters().sym_dequant.fetch_add(1);
-    if (bits == 8) launch_routed<SymW<8>>(g, r, f16, workspace, epilogue, s);
+    if (r.kind == GemmRoute::kDenseRows) {
+        c = rwkv_sym_dequant(qblk, qs, d, workspace, RWKV_F16, OUT, IN, bits, stream);
+        if (c != RWKV_OK) return c;
+        launch_rows(g, workspace, epilogue, s);
+    } else if (bits == 8) launch_routed<SymW<8>>(g, r, f16, workspace, epilogue, s);
     else launch_routed<SymW<6>>(g, r, f16, workspace, epilogue, s);
     RWKV_REQUIRE(hipGetLastError() == hipSuccess, RWKV_E_HIP, "sym_gemm: launch failed");
     rwkv::counters().sym_gemm.fetch_add(1);

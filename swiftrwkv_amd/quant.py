@@ -565,6 +565,17 @@ def rwkvq_gemm_workspace(rows: int, out_features: int, in_features: int) -> int:
     return int(_lib.lib().rwkv_quant_gemm_workspace(rows, out_features, in_features))
 
 
+def rwkvq_gemm_route(kind: str, bits: int, rows: int, out_features: int, in_features: int, out_per: Optional[int] = None,
+                     dtype: torch.dtype = torch.float16, workspace: Optional[int] = None) -> tuple:
+    """The kernel a long-pass GEMM takes: (name, tile rows, tile features, parts K is split over), for kind "sb6"
+    (bits = xbits) or "sym", inputs of `dtype` and `workspace` bytes (None: all it asks for; -1: none)."""
+    ws = rwkvq_gemm_workspace(rows, out_features, in_features) if workspace is None else workspace
+    r = np.zeros(4, np.int32)
+    _lib.call("rwkv_quant_gemm_route", int(kind == "sym"), bits, _OUT_DT[dtype], rows, out_features, in_features,
+              out_per or out_features, ws, r.ctypes.data)
+    return (("ranges", "waves", "dense", "dense rows")[r[0]], int(r[1]), int(r[2]), int(r[3]))
+
+
 def _quant_gemm(entry: str, what: str, x, bufs, out_features: int, in_features: int, code_bits: int, per: int,
                 epilogue: str, out: Optional[torch.Tensor], split: bool = True) -> torch.Tensor:
     G = out_features // per

@@ -75,3 +75,31 @@ def test_quant_gemm_routes(fmt, M, OUT, IN, G):
                      IN, bits, per, 1, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
     assert torch.equal(out[:, :OUT], base[:, :OUT] + y)
     assert torch.equal(out[:, OUT:], base[:, OUT:])
+
+
+@pytest.mark.parametrize("fmt", ["sb6:0", "sb6:1", "sb6:2", "sym:8", "sym:6"])
+@pytest.mark.parametrize("M,OUT,IN,G,kernel,parts", [
+    (65, 16640, 768, 1, "ranges", 3), (128, 16512, 1792, 3, "ranges", 3),
+    (300, 12288, 256, 3, "ranges", 1),
+    (700, 11008, 256, 1, "dense rows", 1), (2000, 4608, 512, 3, "dense rows", 1)])
+def test_ranges_and_row_major_routes(fmt, M, OUT, IN, G, kernel, parts):
+    """K ranges on 128-row tiles and the row-major dense route: each output as test_quant_gemm_routes has it, and bitwise
+    the one-range result where K is not split."""
+    print(f"[case] gemm route {kernel} {fmt} M={M} {OUT}x{IN} G={G}", flush=True)
+    bufs, gemm, entry, bits, w16 = matrix(fmt, OUT, IN, M + OUT)
+    per = OUT // G
+    assert Q.rwkvq_gemm_route(fmt[:3], bits, M, OUT, IN, per)[::3] == (kernel, parts)
+    gen = torch.Generator(device=DEV).manual_seed(M + IN)
+    x = torch.randn((G, M, IN), generator=gen, device=DEV).half()
+    y = gemm(x, *bufs, OUT, IN, bits, out_per=per)
+    assert torch.equal(gemm(x.float(), *bufs, OUT, IN, bits, out_per=per), y)
+    if parts == 1:
+        assert torch.equal(gemm(x, *bufs, OUT, IN, bits, out_per=per, split=False), y)
+    else:
+        for g in range(G):
+            xs, ws, got = x[g].double(), w16[g * per:(g + 1) * per].double(), y[:, g * per:(g + 1) * per]
+            check_f16_rounding(got.cpu().numpy(), (xs @ ws.T).cpu().numpy(), (xs.abs() @ ws.abs().T).cpu().numpy())
+    h = gemm(x, *bufs, OUT, IN, bits, out_per=per, epilogue="relu2_f16")
+    assert torch.equal(h, (torch.relu(y) * torch.relu(y)).half())
+    base = torch.randn((M, OUT), generator=gen, device=DEV)
+    assert torch.equal(gemm(x, *bufs, OUT, IN, bits, out_per=per, epilogue="add", out=base.clone()), base + y)

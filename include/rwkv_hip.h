@@ -318,8 +318,11 @@ rwkv_status rwkv_sym_gemv_ep(const float* x, int64_t N,
  * epilogue 0 stores, 1 adds into y (fp32; the residual update), 2 stores
  * relu(·)² as fp16 (y is then an fp16 buffer; cmix's key, exact in fp16).
  * workspace: NULL, or device memory of rwkv_quant_gemm_workspace(M, OUT, IN)
- * bytes (16-byte aligned; a smaller one is refused before any launch).  With
- * it, passes of few output tiles split the K sum over the waves of a workgroup
+ * bytes, 16-byte aligned.  (A smaller one limits the choice of kernel, and is
+ * refused before any launch where it is also less than the fp16 weight, for 128
+ * or more output tiles of 256 x 256, or than S = min(ceil(384 / tiles), IN /
+ * 192) ranges' fp32 sums, for 2 <= S and fewer than 160 tiles of 128 x 128.)
+ * With it, passes of few output tiles split the K sum over the waves of a workgroup
  * or over ranges whose sums a second launch adds (a fixed order: deterministic,
  * the same bound), and larger ones dequantise the weight into the workspace
  * (fp16) and multiply from there — the same products in the same order as one
@@ -333,9 +336,20 @@ rwkv_status rwkv_sb6_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda
                           int64_t OUT, int64_t IN, int xbits, int64_t out_per, int epilogue, void* workspace,
                           int64_t workspace_bytes, void* stream);
 
+/* rwkv_sb6_gemm with any workspace: the fastest kernel that needs no more than
+ * workspace_bytes (NULL: 0).  rwkv_quant_gemm_auto_workspace (sym 0, bits =
+ * xbits; sym 1 for rwkv_sym_gemm_auto) tells what the fastest of all needs: OUT·IN·2
+ * for a dense route, the sums of K ranges, 0 for the split over waves that
+ * short passes take. */
+int64_t rwkv_quant_gemm_auto_workspace(int sym, int bits, int64_t M, int64_t OUT, int64_t IN, int64_t out_per);
+rwkv_status rwkv_sb6_gemm_auto(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda, int64_t x_group_stride,
+                               const uint8_t* qblk, const uint8_t* qsqm, const uint16_t* ddm, void* y, int64_t ldy,
+                               int64_t OUT, int64_t IN, int xbits, int64_t out_per, int epilogue, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+
 /* Which kernel rwkv_sb6_gemm (sym 0; bits = xbits) or rwkv_sym_gemm (sym 1)
  * takes for a pass with contiguous rows (lda = IN) and this much workspace (< 0:
- * NULL), as four ints: {0, tile rows, tile features, K ranges}, {1, tile rows,
+ * NULL; the _auto entries: 0 for NULL), as four ints: {0, tile rows, tile features, K ranges}, {1, tile rows,
  * tile features (of f16 inputs), waves that split K}, {2, ...} a dequant in the
  * matrix cores' order and a dense product, {3, ...} a row-major dequant and
  * rwkv_f16_gemm's kernel.  Host only. */
@@ -352,6 +366,10 @@ rwkv_status rwkv_sym_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda
                           const uint8_t* qblk, const uint8_t* qs, const uint16_t* d, void* y, int64_t ldy,
                           int64_t OUT, int64_t IN, int bits, int64_t out_per, int epilogue, void* workspace,
                           int64_t workspace_bytes, void* stream);
+rwkv_status rwkv_sym_gemm_auto(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda, int64_t x_group_stride,
+                               const uint8_t* qblk, const uint8_t* qs, const uint16_t* d, void* y, int64_t ldy,
+                               int64_t OUT, int64_t IN, int bits, int64_t out_per, int epilogue, void* workspace,
+                               int64_t workspace_bytes, void* stream);
 
 /* The long pass's fp16 matmul on a dense fp16 weight w [OUT][IN] (K
  * contiguous; the fp16 matmul of baseMatmul once the weight is dequantised,

@@ -226,9 +226,12 @@ public final class RwkvqDeviceSidecar {
                                 inFeatures: info.inFeatures, bits: info.bits)
     }
 
-    /// The workspace a long pass of M rows takes (nil: one K range without).
+    /// The workspace a long pass of M rows uses (nil: none).
     private func gemmWorkspace(_ M: Int, _ info: RwkvqTensorInfo) throws -> (DeviceArray?, Int64) {
-        let n = rwkv_quant_gemm_workspace(Int64(M), Int64(info.outFeatures), Int64(info.inFeatures))
+        let sym = info.kind == .sym
+        let n = rwkv_quant_gemm_auto_workspace(sym ? 1 : 0, Int32(sym ? info.bits : info.xbits), Int64(M),
+                                               Int64(info.outFeatures), Int64(info.inFeatures),
+                                               Int64(info.outFeatures))
         return n > 0 ? (try DeviceArray(shape: [Int(n)], dtype: .uint8), n) : (nil, 0)
     }
 
@@ -244,10 +247,10 @@ public final class RwkvqDeviceSidecar {
         let M = x.shape[0]
         let y = try DeviceArray(shape: [M, info.outFeatures], dtype: .float32)
         let (ws, wsBytes) = try gemmWorkspace(M, info)
-        try check(rwkv_sb6_gemm(x.raw, x.dtype.code, Int64(M), Int64(info.inFeatures), Int64(M * info.inFeatures),
-                                qblk.u8, qsqm.u8, ddm.u16, y.raw, Int64(info.outFeatures), Int64(info.outFeatures),
-                                Int64(info.inFeatures), Int32(info.xbits), Int64(info.outFeatures), 0,
-                                ws?.raw, wsBytes, streamArg))
+        try check(rwkv_sb6_gemm_auto(x.raw, x.dtype.code, Int64(M), Int64(info.inFeatures), Int64(M * info.inFeatures),
+                                     qblk.u8, qsqm.u8, ddm.u16, y.raw, Int64(info.outFeatures), Int64(info.outFeatures),
+                                     Int64(info.inFeatures), Int32(info.xbits), Int64(info.outFeatures), 0,
+                                     ws?.raw, wsBytes, streamArg))
         return y
     }
 
@@ -262,10 +265,10 @@ public final class RwkvqDeviceSidecar {
         let M = x.shape[0]
         let y = try DeviceArray(shape: [M, info.outFeatures], dtype: .float32)
         let (ws, wsBytes) = try gemmWorkspace(M, info)
-        try check(rwkv_sym_gemm(x.raw, x.dtype.code, Int64(M), Int64(info.inFeatures), Int64(M * info.inFeatures),
-                                qblk.u8, qs.u8, d.u16, y.raw, Int64(info.outFeatures), Int64(info.outFeatures),
-                                Int64(info.inFeatures), Int32(info.bits), Int64(info.outFeatures), 0,
-                                ws?.raw, wsBytes, streamArg))
+        try check(rwkv_sym_gemm_auto(x.raw, x.dtype.code, Int64(M), Int64(info.inFeatures), Int64(M * info.inFeatures),
+                                     qblk.u8, qs.u8, d.u16, y.raw, Int64(info.outFeatures), Int64(info.outFeatures),
+                                     Int64(info.inFeatures), Int32(info.bits), Int64(info.outFeatures), 0,
+                                     ws?.raw, wsBytes, streamArg))
         return y
     }
 }

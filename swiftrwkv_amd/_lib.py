@@ -98,7 +98,10 @@ _SIGS = {
     "rwkv_sym_gemv_ep": (I, [P, L, P, P, P, P, L, L, I, I, P]),
     "rwkv_sb6_gemm_applies": (I, [L, L, I, L]),
     "rwkv_sb6_gemm": (I, [P, I, L, L, L, P, P, P, P, L, L, L, I, L, I, P, L, P]),
+    "rwkv_sb6_gemm_auto": (I, [P, I, L, L, L, P, P, P, P, L, L, L, I, L, I, P, L, P]),
+    "rwkv_sym_gemm_auto": (I, [P, I, L, L, L, P, P, P, P, L, L, L, I, L, I, P, L, P]),
     "rwkv_quant_gemm_workspace": (L, [L, L, L]),
+    "rwkv_quant_gemm_auto_workspace": (L, [I, I, L, L, L, L]),
     "rwkv_quant_gemm_route": (I, [I, I, I, L, L, L, L, L, P]),
     "rwkv_f16_gemm_applies": (I, [L, L, L, L]),
     "rwkv_f16_gemm": (I, [P, L, L, L, P, P, L, L, L, L, I, P]),

@@ -1220,10 +1220,10 @@ GemmRoute gemm_route(int fmt, int64_t M, int64_t N, int64_t K, int64_t out_per, 
     return best;
 }
 
-// Bytes of workspace a pass of this shape takes, whatever the format.  The
-// split over waves needs none of its own; it asks for two ranges' fp32 sums,
-// the least that a caller's workspace for such a shape has held, so that the
-// size still tells which shapes want one.
+// Bytes of workspace that let a pass of this shape take its fastest route,
+// whatever the format, for the entry points where NULL means one range: the
+// split over waves touches none and asks for two ranges' fp32 sums, so that no
+// shape that has a faster route is taken for one that has not.
 int64_t gemm_workspace(int64_t M, int64_t N, int64_t K) {
     int64_t need = 0;
     for (int f = 0; f < kFormats; ++f) {
@@ -1382,26 +1382,105 @@ rwkv_status gemm_check(const char* who, const void* x, rwkv_dtype x_dt, int64_t 
     return RWKV_OK;
 }
 
-// A caller's workspace: NULL, or at least rwkv_quant_gemm_workspace bytes,
-// 16-byte aligned (checked before anything is launched).
-rwkv_status gemm_workspace_check(const char* who, int64_t M, int64_t N, int64_t K, const void* workspace,
-                                 int64_t workspace_bytes) {
-    if (workspace == nullptr) return RWKV_OK;
-    const int64_t need = gemm_workspace(M, N, K);
-    RWKV_REQUIRE(workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0, RWKV_E_SHAPE,
-                 "%s: workspace of %lld bytes (16-byte aligned) needed, %lld given", who, (long long)need,
+// A caller's workspace (checked before anything is launched): 16-byte aligned;
+// `least` is what is refused below.
+rwkv_status gemm_workspace_check(const char* who, int64_t least, const void* workspace, int64_t workspace_bytes) {
+    RWKV_REQUIRE(workspace_bytes >= least && reinterpret_cast<uintptr_t>(workspace) % 16 == 0, RWKV_E_SHAPE,
+                 "%s: workspace of %lld bytes (16-byte aligned) needed, %lld given", who, (long long)least,
                  (long long)workspace_bytes);
     return RWKV_OK;
 }
 
-// The route of an entry's call: one K range without a workspace.
+// The least workspace of the entry points where NULL means one range: what
+// gemm_workspace asks for, or what a caller may have sized by another rule, if
+// that is less — the fp16 weight from 128 tiles of 256 × 256, else the sums of
+// the K ranges that 128 × 128 tiles are split into, nothing for one range.  The
+// route keeps within the bytes given.
+int64_t gemm_workspace_least(int64_t M, int64_t N, int64_t K) {
+    const int64_t S = gemm_splits(M, N, K);
+    const bool dense = dense_shape_ok(M, N, K, N, K) && ((M + DT - 1) / DT) * (N / DT) >= 128;
+    const int64_t other = dense ? N * K * 2 : S > 1 ? S * M * N * 4 : 0;
+    return other ? std::min(other, gemm_workspace(M, N, K)) : 0;
+}
+
+// Route of a call with this much workspace (< 0: one K range).
 GemmRoute entry_route(int fmt, rwkv_dtype x_dt, int64_t M, int64_t N, int64_t K, int64_t out_per, int64_t lda,
-                      const void* workspace, int64_t workspace_bytes) {
+                      int64_t workspace_bytes) {
     GemmRoute r;
-    if (workspace) r = gemm_route(fmt, M, N, K, out_per, lda, workspace_bytes);
+    if (workspace_bytes >= 0) r = gemm_route(fmt, M, N, K, out_per, lda, workspace_bytes);
     // row-major weights meet fp16 inputs only; operand order gives the same bits
     if (r.kind == GemmRoute::kDenseRows && x_dt != RWKV_F16) r.kind = GemmRoute::kDense;
     return r;
+}
+
+// The workspace an entry's call routes with: what NULL means is all that sets
+// rwkv_*_gemm (one range) and rwkv_*_gemm_auto (no workspace) apart.
+rwkv_status entry_workspace(const char* who, bool any, int64_t M, int64_t N, int64_t K, const void* workspace,
+                            int64_t* workspace_bytes) {
+    if (workspace == nullptr) {
+        *workspace_bytes = any ? 0 : -1;
+        return RWKV_OK;
+    }
+    return gemm_workspace_check(who, any ? 0 : gemm_workspace_least(M, N, K), workspace, *workspace_bytes);
+}
+
+rwkv_status sb6_gemm(const char* who, bool any, const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda,
+                     int64_t x_group_stride, const uint8_t* qblk, const uint8_t* qsqm, const uint16_t* ddm, void* y,
+                     int64_t ldy, int64_t OUT, int64_t IN, int xbits, int64_t out_per, int epilogue, void* workspace,
+                     int64_t workspace_bytes, void* stream) {
+    RWKV_REQUIRE(x && qblk && qsqm && ddm && y, RWKV_E_NULL, "%s: null buffer", who);
+    RWKV_REQUIRE(rwkv_sb6_gemm_applies(OUT, IN, xbits, out_per), RWKV_E_UNSUPPORTED,
+                 "%s: xbits %d (0..2), OUT (%lld) and out_per (%lld) multiples of 128, IN (%lld) of 256", who, xbits,
+                 (long long)OUT, (long long)out_per, (long long)IN);
+    rwkv_status c = gemm_check(who, x, x_dt, M, lda, x_group_stride, ldy, OUT, IN, out_per, epilogue);
+    if (c != RWKV_OK) return c;
+    c = entry_workspace(who, any, M, OUT, IN, workspace, &workspace_bytes);
+    if (c != RWKV_OK) return c;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const GemmArgs g{x, lda, x_group_stride, qblk, qsqm, ddm, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per, nullptr, 1};
+    const bool f16 = x_dt == RWKV_F16;
+    const GemmRoute r = entry_route(kSb6 + xbits, x_dt, M, OUT, IN, out_per, lda, workspace_bytes);
+    if (r.kind == GemmRoute::kDense) rwkv::counters().sb6_dequant.fetch_add(1);
+    if (r.kind == GemmRoute::kDenseRows) {
+        c = rwkv_sb6_dequant(qblk, qsqm, ddm, workspace, RWKV_F16, OUT, IN, xbits, stream);
+        if (c != RWKV_OK) return c;
+        launch_rows(g, workspace, epilogue, s);
+    } else if (xbits == 0) launch_routed<Sb6W<0>>(g, r, f16, workspace, epilogue, s);
+    else if (xbits == 1) launch_routed<Sb6W<1>>(g, r, f16, workspace, epilogue, s);
+    else launch_routed<Sb6W<2>>(g, r, f16, workspace, epilogue, s);
+    RWKV_REQUIRE(hipGetLastError() == hipSuccess, RWKV_E_HIP, "%s: launch failed", who);
+    rwkv::counters().sb6_gemm.fetch_add(1);
+    rwkv::clear_error();
+    return RWKV_OK;
+}
+
+rwkv_status sym_gemm(const char* who, bool any, const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda,
+                     int64_t x_group_stride, const uint8_t* qblk, const uint8_t* qs, const uint16_t* d, void* y,
+                     int64_t ldy, int64_t OUT, int64_t IN, int bits, int64_t out_per, int epilogue, void* workspace,
+                     int64_t workspace_bytes, void* stream) {
+    RWKV_REQUIRE(x && qblk && qs && d && y, RWKV_E_NULL, "%s: null buffer", who);
+    RWKV_REQUIRE(rwkv_sym_gemm_applies(OUT, IN, bits, out_per), RWKV_E_UNSUPPORTED,
+                 "%s: %d-bit codes (8 or 6), OUT (%lld) and out_per (%lld) multiples of 128, IN (%lld) of 256", who,
+                 bits, (long long)OUT, (long long)out_per, (long long)IN);
+    rwkv_status c = gemm_check(who, x, x_dt, M, lda, x_group_stride, ldy, OUT, IN, out_per, epilogue);
+    if (c != RWKV_OK) return c;
+    c = entry_workspace(who, any, M, OUT, IN, workspace, &workspace_bytes);
+    if (c != RWKV_OK) return c;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const GemmArgs g{x, lda, x_group_stride, qblk, qs, d, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per, nullptr, 1};
+    const bool f16 = x_dt == RWKV_F16;
+    const GemmRoute r = entry_route(bits == 8 ? kSym8 : kSym6, x_dt, M, OUT, IN, out_per, lda, workspace_bytes);
+    if (r.kind == GemmRoute::kDense) rwkv::counters().sym_dequant.fetch_add(1);
+    if (r.kind == GemmRoute::kDenseRows) {
+        c = rwkv_sym_dequant(qblk, qs, d, workspace, RWKV_F16, OUT, IN, bits, stream);
+        if (c != RWKV_OK) return c;
+        launch_rows(g, workspace, epilogue, s);
+    } else if (bits == 8) launch_routed<SymW<8>>(g, r, f16, workspace, epilogue, s);
+    else launch_routed<SymW<6>>(g, r, f16, workspace, epilogue, s);
+    RWKV_REQUIRE(hipGetLastError() == hipSuccess, RWKV_E_HIP, "%s: launch failed", who);
+    rwkv::counters().sym_gemm.fetch_add(1);
+    rwkv::clear_error();
+    return RWKV_OK;
 }
 
 }  // namespace
@@ -1417,13 +1496,21 @@ rwkv_status rwkv_quant_gemm_route(int sym, int bits, rwkv_dtype x_dt, int64_t M,
     RWKV_REQUIRE(M >= 1 && M <= ((int64_t)1 << 24), RWKV_E_SHAPE, "quant_gemm_route: M (%lld) out of range", (long long)M);
     RWKV_REQUIRE(x_dt == RWKV_F32 || x_dt == RWKV_F16, RWKV_E_DTYPE, "quant_gemm_route: inputs are f32 or f16");
     const GemmRoute r = entry_route(sym ? (bits == 8 ? kSym8 : kSym6) : kSb6 + bits, x_dt, M, OUT, IN, out_per, IN,
-                                    workspace_bytes < 0 ? nullptr : route, workspace_bytes);
+                                    workspace_bytes);
     route[0] = r.kind;
     route[1] = r.kind == GemmRoute::kDenseRows ? DT : r.tm;
     route[2] = r.kind == GemmRoute::kDenseRows ? DT : r.tn;
     route[3] = r.parts;
     rwkv::clear_error();
     return RWKV_OK;
+}
+
+int64_t rwkv_quant_gemm_auto_workspace(int sym, int bits, int64_t M, int64_t OUT, int64_t IN, int64_t out_per) {
+    if (M < 1 || M > ((int64_t)1 << 24) ||
+        !(sym ? rwkv_sym_gemm_applies(OUT, IN, bits, out_per) : rwkv_sb6_gemm_applies(OUT, IN, bits, out_per)))
+        return 0;
+    const int fmt = sym ? (bits == 8 ? kSym8 : kSym6) : kSb6 + bits;
+    return route_bytes(gemm_route(fmt, M, OUT, IN, out_per, IN, INT64_MAX), M, OUT, IN);
 }
 
 int64_t rwkv_quant_gemm_workspace(int64_t M, int64_t OUT, int64_t IN) {
@@ -1439,30 +1526,16 @@ rwkv_status rwkv_sb6_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda
                           const uint8_t* qblk, const uint8_t* qsqm, const uint16_t* ddm, void* y, int64_t ldy,
                           int64_t OUT, int64_t IN, int xbits, int64_t out_per, int epilogue, void* workspace,
                           int64_t workspace_bytes, void* stream) {
-    RWKV_REQUIRE(x && qblk && qsqm && ddm && y, RWKV_E_NULL, "sb6_gemm: null buffer");
-    RWKV_REQUIRE(rwkv_sb6_gemm_applies(OUT, IN, xbits, out_per), RWKV_E_UNSUPPORTED,
-                 "sb6_gemm: xbits %d (0..2), OUT (%lld) and out_per (%lld) multiples of 128, IN (%lld) of 256", xbits,
-                 (long long)OUT, (long long)out_per, (long long)IN);
-    rwkv_status c = gemm_check("sb6_gemm", x, x_dt, M, lda, x_group_stride, ldy, OUT, IN, out_per, epilogue);
-    if (c != RWKV_OK) return c;
-    c = gemm_workspace_check("sb6_gemm", M, OUT, IN, workspace, workspace_bytes);
-    if (c != RWKV_OK) return c;
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const GemmArgs g{x, lda, x_group_stride, qblk, qsqm, ddm, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per, nullptr, 1};
-    const bool f16 = x_dt == RWKV_F16;
-    const GemmRoute r = entry_route(kSb6 + xbits, x_dt, M, OUT, IN, out_per, lda, workspace, workspace_bytes);
-    if (r.kind == GemmRoute::kDense) rwkv::counters().sb6_dequant.fetch_add(1);
-    if (r.kind == GemmRoute::kDenseRows) {
-        c = rwkv_sb6_dequant(qblk, qsqm, ddm, workspace, RWKV_F16, OUT, IN, xbits, stream);
-        if (c != RWKV_OK) return c;
-        launch_rows(g, workspace, epilogue, s);
-    } else if (xbits == 0) launch_routed<Sb6W<0>>(g, r, f16, workspace, epilogue, s);
-    else if (xbits == 1) launch_routed<Sb6W<1>>(g, r, f16, workspace, epilogue, s);
-    else launch_routed<Sb6W<2>>(g, r, f16, workspace, epilogue, s);
-    RWKV_REQUIRE(hipGetLastError() == hipSuccess, RWKV_E_HIP, "sb6_gemm: launch failed");
-    rwkv::counters().sb6_gemm.fetch_add(1);
-    rwkv::clear_error();
-    return RWKV_OK;
+    return sb6_gemm("sb6_gemm", false, x, x_dt, M, lda, x_group_stride, qblk, qsqm, ddm, y, ldy, OUT, IN, xbits, out_per,
+                    epilogue, workspace, workspace_bytes, stream);
+}
+
+rwkv_status rwkv_sb6_gemm_auto(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda, int64_t x_group_stride,
+                               const uint8_t* qblk, const uint8_t* qsqm, const uint16_t* ddm, void* y, int64_t ldy,
+                               int64_t OUT, int64_t IN, int xbits, int64_t out_per, int epilogue, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+    return sb6_gemm("sb6_gemm_auto", true, x, x_dt, M, lda, x_group_stride, qblk, qsqm, ddm, y, ldy, OUT, IN, xbits, out_per,
+                    epilogue, workspace, workspace_bytes, stream);
 }
 
 int rwkv_sym_gemm_applies(int64_t OUT, int64_t IN, int bits, int64_t out_per) {
@@ -1473,29 +1546,16 @@ rwkv_status rwkv_sym_gemm(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda
                           const uint8_t* qblk, const uint8_t* qs, const uint16_t* d, void* y, int64_t ldy,
                           int64_t OUT, int64_t IN, int bits, int64_t out_per, int epilogue, void* workspace,
                           int64_t workspace_bytes, void* stream) {
-    RWKV_REQUIRE(x && qblk && qs && d && y, RWKV_E_NULL, "sym_gemm: null buffer");
-    RWKV_REQUIRE(rwkv_sym_gemm_applies(OUT, IN, bits, out_per), RWKV_E_UNSUPPORTED,
-                 "sym_gemm: %d-bit codes (8 or 6), OUT (%lld) and out_per (%lld) multiples of 128, IN (%lld) of 256",
-                 bits, (long long)OUT, (long long)out_per, (long long)IN);
-    rwkv_status c = gemm_check("sym_gemm", x, x_dt, M, lda, x_group_stride, ldy, OUT, IN, out_per, epilogue);
-    if (c != RWKV_OK) return c;
-    c = gemm_workspace_check("sym_gemm", M, OUT, IN, workspace, workspace_bytes);
-    if (c != RWKV_OK) return c;
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const GemmArgs g{x, lda, x_group_stride, qblk, qs, d, y, ldy, (int)M, (int)OUT, (int)IN, (int)out_per, nullptr, 1};
-    const bool f16 = x_dt == RWKV_F16;
-    const GemmRoute r = entry_route(bits == 8 ? kSym8 : kSym6, x_dt, M, OUT, IN, out_per, lda, workspace, workspace_bytes);
-    if (r.kind == GemmRoute::kDense) rwkv::counters().sym_dequant.fetch_add(1);
-    if (r.kind == GemmRoute::kDenseRows) {
-        c = rwkv_sym_dequant(qblk, qs, d, workspace, RWKV_F16, OUT, IN, bits, stream);
-        if (c != RWKV_OK) return c;
-        launch_rows(g, workspace, epilogue, s);
-    } else if (bits == 8) launch_routed<SymW<8>>(g, r, f16, workspace, epilogue, s);
-    else launch_routed<SymW<6>>(g, r, f16, workspace, epilogue, s);
-    RWKV_REQUIRE(hipGetLastError() == hipSuccess, RWKV_E_HIP, "sym_gemm: launch failed");
-    rwkv::counters().sym_gemm.fetch_add(1);
-    rwkv::clear_error();
-    return RWKV_OK;
+    return sym_gemm("sym_gemm", false, x, x_dt, M, lda, x_group_stride, qblk, qs, d, y, ldy, OUT, IN, bits, out_per,
+                    epilogue, workspace, workspace_bytes, stream);
+}
+
+rwkv_status rwkv_sym_gemm_auto(const void* x, rwkv_dtype x_dt, int64_t M, int64_t lda, int64_t x_group_stride,
+                               const uint8_t* qblk, const uint8_t* qs, const uint16_t* d, void* y, int64_t ldy,
+                               int64_t OUT, int64_t IN, int bits, int64_t out_per, int epilogue, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+    return sym_gemm("sym_gemm_auto", true, x, x_dt, M, lda, x_group_stride, qblk, qs, d, y, ldy, OUT, IN, bits, out_per,
+                    epilogue, workspace, workspace_bytes, stream);
 }
 
 int rwkv_f16_gemm_applies(int64_t M, int64_t OUT, int64_t IN, int64_t out_per) {

@@ -560,23 +560,31 @@ _GEMM_EP = {"store": 0, "add": 1, "relu2_f16": 2}
 
 
 def rwkvq_gemm_workspace(rows: int, out_features: int, in_features: int) -> int:
-    """Bytes of the workspace a long-pass GEMM of this shape wants (0: it runs as
-    one K range without; the C entry runs any shape so when given none)."""
+    """Bytes of the workspace rwkv_sb6_gemm / rwkv_sym_gemm want for a pass of this
+    shape (they run it as one K range when given none; the wrappers here take
+    rwkvq_gemm_auto_workspace's bytes)."""
     return int(_lib.lib().rwkv_quant_gemm_workspace(rows, out_features, in_features))
+
+
+def rwkvq_gemm_auto_workspace(kind: str, bits: int, rows: int, out_features: int, in_features: int,
+                              out_per: Optional[int] = None) -> int:
+    """Bytes of workspace the fastest kernel of this pass uses (kind "sb6", bits = xbits, or "sym")."""
+    return int(_lib.lib().rwkv_quant_gemm_auto_workspace(int(kind == "sym"), bits, rows, out_features, in_features,
+                                                         out_per or out_features))
 
 
 def rwkvq_gemm_route(kind: str, bits: int, rows: int, out_features: int, in_features: int, out_per: Optional[int] = None,
                      dtype: torch.dtype = torch.float16, workspace: Optional[int] = None) -> tuple:
     """The kernel a long-pass GEMM takes: (name, tile rows, tile features, parts K is split over), for kind "sb6"
-    (bits = xbits) or "sym", inputs of `dtype` and `workspace` bytes (None: all it asks for; -1: none)."""
-    ws = rwkvq_gemm_workspace(rows, out_features, in_features) if workspace is None else workspace
+    (bits = xbits) or "sym", inputs of `dtype` and `workspace` bytes (None: all it asks for; -1: one K range)."""
+    ws = (1 << 62) if workspace is None else workspace
     r = np.zeros(4, np.int32)
     _lib.call("rwkv_quant_gemm_route", int(kind == "sym"), bits, _OUT_DT[dtype], rows, out_features, in_features,
               out_per or out_features, ws, r.ctypes.data)
     return (("ranges", "waves", "dense", "dense rows")[r[0]], int(r[1]), int(r[2]), int(r[3]))
 
 
-def _quant_gemm(entry: str, what: str, x, bufs, out_features: int, in_features: int, code_bits: int, per: int,
+def _quant_gemm(what: str, x, bufs, out_features: int, in_features: int, code_bits: int, per: int,
                 epilogue: str, out: Optional[torch.Tensor], split: bool = True) -> torch.Tensor:
     G = out_features // per
     if x.dim() == 2:
@@ -596,9 +604,10 @@ def _quant_gemm(entry: str, what: str, x, bufs, out_features: int, in_features: 
     elif out.dtype != ydt or tuple(out.shape) != (M, out_features) or not out.is_contiguous() or \
             out.device != x.device:
         raise ValueError(f"{what} GEMM: out must be a contiguous {ydt} [{M}, {out_features}] tensor on {x.device}")
-    need = rwkvq_gemm_workspace(M, out_features, in_features) if split else 0
+    L = _lib.lib()
+    need = L.rwkv_quant_gemm_auto_workspace(what == "sym", code_bits, M, out_features, in_features, per) if split else 0
     ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
-    _lib.call(entry, x.data_ptr(), _OUT_DT[x.dtype], M, in_features, M * in_features, *[b.data_ptr() for b in bufs],
+    _lib.call(f"rwkv_{what}_gemm_auto" if split else f"rwkv_{what}_gemm", x.data_ptr(), _OUT_DT[x.dtype], M, in_features, M * in_features, *[b.data_ptr() for b in bufs],
               out.data_ptr(), out_features, out_features, in_features, code_bits, per, ep,
               ws.data_ptr() if need else None, need, _stream(x))
     return out
@@ -612,14 +621,14 @@ def rwkvq_sb6_gemm(x, qblk, qsqm, ddm, out_features: int, in_features: int, xbit
     [M, OUT] = fp16(fp16(x)·fp16(W)ᵀ) with fp32 sums.  x [M, IN] (one matrix)
     or [G, M, IN] (G = OUT / out_per row-concatenated matrices, matrix g
     reading x[g]), fp32 or fp16.  epilogue "store" / "add" (fp32 `out`, added
-    into) / "relu2_f16" (relu(·)² in an fp16 `out`).  `split`: take the kernels
-    that want a workspace (one per call), some of which sum K in ranges (False:
-    one range)."""
+    into) / "relu2_f16" (relu(·)² in an fp16 `out`).  `split`: the fastest
+    kernel, some of which split the K sum or use a workspace (made per call);
+    False: one K range."""
     per = out_features if out_per is None else out_per
     if not rwkvq_sb6_gemm_applies(out_features, in_features, xbits, per):
         raise ValueError(f"sb6 GEMM: [{out_features}, {in_features}] xbits={xbits} out_per={per} not taken")
     bufs = _sb6_bufs(qblk, qsqm, ddm, out_features, in_features, xbits)
-    return _quant_gemm("rwkv_sb6_gemm", "sb6", x, bufs, out_features, in_features, xbits, per, epilogue, out, split)
+    return _quant_gemm("sb6", x, bufs, out_features, in_features, xbits, per, epilogue, out, split)
 
 
 def rwkvq_sym_gemm(x, qblk, qs, d, out_features: int, in_features: int, bits: int,
@@ -632,7 +641,7 @@ def rwkvq_sym_gemm(x, qblk, qs, d, out_features: int, in_features: int, bits: in
     if not rwkvq_sym_gemm_applies(out_features, in_features, bits, per):
         raise ValueError(f"sym GEMM: [{out_features}, {in_features}] bits={bits} out_per={per} not taken")
     bufs = _sym_bufs(qblk, qs, d, out_features, in_features, bits)
-    return _quant_gemm("rwkv_sym_gemm", "sym", x, bufs, out_features, in_features, bits, per, epilogue, out, split)
+    return _quant_gemm("sym", x, bufs, out_features, in_features, bits, per, epilogue, out, split)
 
 
 def rwkvq_f16_gemm_applies(rows: int, out_features: int, in_features: int, out_per: Optional[int] = None) -> bool:

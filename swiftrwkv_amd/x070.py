@@ -450,7 +450,7 @@ class X070Decoder:
     batch_mfma: Optional[bool] = None
 
     def _batch_ws(self, nbytes: int) -> torch.Tensor:
-        """The workspace the batched GEMV and the split long-pass GEMM share
+        """The workspace the batched GEMV and the long-pass GEMM share
         (their launches are ordered on the stream), grown when a call needs more.
         A grown-out buffer is kept alive (not returned to the caching
         allocator): a HIP graph captured through launch() before the growth
@@ -873,16 +873,17 @@ class X070Decoder:
 
     def _long_gemm(self, q, xp, xdt, M, yp, ldy, ep, s) -> bool:
         """One matrix (group) of the long pass on the matrix cores, when the
-        kernels take its layout; False otherwise (nothing launched).  Shapes
-        with few output tiles split their K sum in the shared workspace."""
+        kernels take its layout; False otherwise (nothing launched).  Kernels
+        that need one (a dequantised weight, sums of K ranges) use the shared
+        workspace."""
         L = _lib.lib()
         if q.kind == "sb6" and L.rwkv_sb6_gemm_applies(q.OUT, q.IN, q.xbits, q.out_per):
-            entry, bits = L.rwkv_sb6_gemm, q.xbits
+            entry, sym, bits = L.rwkv_sb6_gemm_auto, 0, q.xbits
         elif q.kind == "sym" and L.rwkv_sym_gemm_applies(q.OUT, q.IN, q.bits, q.out_per):
-            entry, bits = L.rwkv_sym_gemm, q.bits
+            entry, sym, bits = L.rwkv_sym_gemm_auto, 1, q.bits
         else:
             return False
-        need = int(L.rwkv_quant_gemm_workspace(M, q.OUT, q.IN))
+        need = int(L.rwkv_quant_gemm_auto_workspace(sym, bits, M, q.OUT, q.IN, q.out_per))
         ws = self._batch_ws(need).data_ptr() if need else None
         _lib.check(entry(xp, xdt, M, q.IN, M * q.IN, q.bufs[0].data_ptr(), q.bufs[1].data_ptr(), q.bufs[2].data_ptr(),
                          yp, ldy, q.OUT, q.IN, bits, q.out_per, ep, ws, need, s))

@@ -35,9 +35,9 @@ def test_route_fits_its_workspace_and_its_inputs(kind, bits):
     for M in (1, 40, 65, 100, 128, 300, 1500, 4096, 20000):
         for OUT, IN in ((128, 256), (768, 768), (2304, 256), (4096, 4096), (10240, 5888), (14336, 4096), (16640, 768)):
             for out_per in {OUT, 128} | ({OUT // 3} if OUT % 384 == 0 else set()):
-                for ws in (-1, 0, 16, 8 * M * OUT, OUT * IN * 2, None):
+                for ws in (-1, 0, 16, 8 * M * OUT, OUT * IN * 2, Q.rwkvq_gemm_workspace(M, OUT, IN), None):
                     name, tm, tn, parts = Q.rwkvq_gemm_route(kind, bits, M, OUT, IN, out_per, workspace=ws)
-                    have = Q.rwkvq_gemm_workspace(M, OUT, IN) if ws is None else ws
+                    have = Q.rwkvq_gemm_auto_workspace(kind, bits, M, OUT, IN, out_per) if ws is None else ws
                     need = OUT * IN * 2 if name.startswith("dense") else 4 * parts * M * OUT if name == "ranges" and parts > 1 else 0
                     assert need <= max(have, 0)
                     assert OUT % tn == 0 and (not name.startswith("dense") or out_per % tn == 0)

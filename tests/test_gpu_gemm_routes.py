@@ -103,3 +103,45 @@ def test_ranges_and_row_major_routes(fmt, M, OUT, IN, G, kernel, parts):
     assert torch.equal(h, (torch.relu(y) * torch.relu(y)).half())
     base = torch.randn((M, OUT), generator=gen, device=DEV)
     assert torch.equal(gemm(x, *bufs, OUT, IN, bits, out_per=per, epilogue="add", out=base.clone()), base + y)
+
+
+@pytest.mark.parametrize("fmt,M,OUT,IN", [("sb6:0", 300, 12288, 256), ("sym:6", 300, 12288, 256), ("sb6:2", 1024, 4096, 512)])
+def test_small_workspace_is_taken_where_one_range_fills_the_chip(fmt, M, OUT, IN):
+    """160 or more 128 × 128 tiles, too few 256 × 256 ones for the dense kernel: any aligned workspace runs, by the
+    kernels that fit in it; without one the _auto entry picks among those too."""
+    print(f"[case] gemm small workspace {fmt} M={M} {OUT}x{IN}", flush=True)
+    bufs, gemm, entry, bits, w16 = matrix(fmt, OUT, IN, M + OUT)
+    x = torch.randn((M, IN), generator=torch.Generator(device=DEV).manual_seed(M), device=DEV).half()
+    exact, mag = x.double() @ w16.double().T, x.double().abs() @ w16.double().abs().T
+    ws = torch.zeros(64, dtype=torch.uint8, device=DEV)
+    auto = getattr(_lib.lib(), f"rwkv_{fmt[:3]}_gemm_auto")
+    got = []
+    for f, p, n in ((entry, ws.data_ptr(), 16), (auto, ws.data_ptr(), 16), (auto, None, 0)):
+        y = torch.empty((M, OUT), device=DEV)
+        _lib.check(f(x.data_ptr(), _lib.F16, M, IN, M * IN, *[b.data_ptr() for b in bufs], y.data_ptr(), OUT, OUT, IN, bits,
+                     OUT, 0, p, n, torch.cuda.current_stream().cuda_stream))
+        got.append(y)
+    check_f16_rounding(got[0].cpu().numpy(), exact.cpu().numpy(), mag.cpu().numpy())
+    assert torch.equal(got[1], got[0]) and torch.equal(got[2], got[0])
+    assert not ws.any()
+
+
+@pytest.mark.parametrize("fmt,M,OUT,IN", [("sb6:0", 128, 3072, 768), ("sym:8", 700, 768, 768), ("sym:6", 33, 4096, 4096)])
+def test_wave_split_takes_no_memory(fmt, M, OUT, IN):
+    """A pass split over waves allocates its output and nothing else; its bits are those of a call with a workspace."""
+    print(f"[case] gemm memory {fmt} M={M} {OUT}x{IN}", flush=True)
+    bufs, gemm, entry, bits, _ = matrix(fmt, OUT, IN, M)
+    assert Q.rwkvq_gemm_route(fmt[:3], bits, M, OUT, IN)[0] == "waves"
+    assert Q.rwkvq_gemm_auto_workspace(fmt[:3], bits, M, OUT, IN) == 0
+    x = torch.randn((M, IN), generator=torch.Generator(device=DEV).manual_seed(M), device=DEV).half()
+    out = torch.empty((M, OUT), device=DEV)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    gemm(x, *bufs, OUT, IN, bits, out=out)
+    assert torch.cuda.max_memory_allocated() == before
+    need = Q.rwkvq_gemm_workspace(M, OUT, IN)
+    ws, y = torch.empty(need, dtype=torch.uint8, device=DEV), torch.empty((M, OUT), device=DEV)
+    _lib.check(entry(x.data_ptr(), _lib.F16, M, IN, M * IN, *[b.data_ptr() for b in bufs], y.data_ptr(), OUT, OUT, IN, bits,
+                     OUT, 0, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(y, out)

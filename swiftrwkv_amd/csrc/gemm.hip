@@ -1090,7 +1090,7 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(DenseArgs g) {
 //     × 3072 × 1024 21.7 (32.9), 4096 × 1024 × 4096 44.7 (134).
 //   * the dense route over row-major weights (rwkv_*_dequant +
 //     dense_gemm_kernel; fp16 inputs): one round costs more, but each tile
-//     starts and ends sooner, which tells up to K ~ 1024: 8192 × 3072 × 256
+//     starts and ends sooner, which tells for a short K: 8192 × 3072 × 256
 //     31.9 (37.5 over operand order), 4177 × 12288 × 768 107 (117), 8192 ×
 //     4096 × 1024 77 (78), 4096 × 4096 × 4096 126 (119).
 //   * K ranges on 128 × 128 tiles (quant_gemm_kernel), where a tile's 128 rows
@@ -1200,8 +1200,9 @@ GemmRoute gemm_route(int fmt, int64_t M, int64_t N, int64_t K, int64_t out_per, 
         tile = &t;
     }
     if (tile) offer(tile_cost, {GemmRoute::kDense, tile->tm, tile->tn, 1});
-    // the row-major dequant's thread index is 32-bit
-    if (tile && dense_shape_ok(M, N, K, out_per, lda) && N * (K / 8) < INT32_MAX)
+    // row-major: 4 % faster at K = 1280, the same from 2304 to 4096, 2 % slower
+    // beyond (medians over 1,300 passes); its dequant's thread index is 32-bit
+    if (tile && K <= 2560 && dense_shape_ok(M, N, K, out_per, lda) && N * (K / 8) < INT32_MAX)
         offer(dense(row_major), {GemmRoute::kDenseRows, tile->tm, tile->tn, 1});
 
     const int64_t blocks = ((M + 127) / 128) * (N / 128);

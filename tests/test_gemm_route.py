@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from swiftrwkv_amd import quant as Q
+from tests.test_gpu_gemm_routes import SHAPES
 
 FORMATS = [("sb6", 0), ("sb6", 1), ("sb6", 2), ("sym", 8), ("sym", 6)]
 
@@ -45,3 +46,14 @@ def test_route_fits_its_workspace_and_its_inputs(kind, bits):
                     assert n32 == {"dense rows": "dense"}.get(name, name) and parts32 == parts
                     if ws == -1:
                         assert (name, parts) == ("ranges", 1)
+
+
+def test_gpu_shapes_take_the_kernels_they_are_listed_for():
+    """The GPU tests' shapes (tests/test_gpu_gemm_routes.py) reach every kernel and tile in every format."""
+    listed = [(k, s) for k, v in SHAPES.items() if k for s in v]
+    wrong = [(k, s, f, r) for k, s in listed for f in FORMATS
+             if (r := Q.rwkvq_gemm_route(*f, *s[:3], s[1] // s[3])[:3]) != k]
+    assert not wrong
+    assert {k for k, _ in listed} == {("waves", m, n) for m, n in ((16, 16), (32, 16), (32, 32), (64, 16), (64, 32), (64, 64))} | {
+        ("dense", m, n) for m, n in ((64, 64), (64, 128), (128, 128), (256, 256))} | {("dense rows", 256, 256),
+                                                                                      ("ranges", 128, 128)}

@@ -1,9 +1,10 @@
-"""The kernels a quantised long pass is routed to by its shape (csrc/gemm.hip, gemm_route): the K sum split over a
-workgroup's waves, on every tile, and the dense route over operand-ordered weights, on every tile.
+"""The kernels a quantised long pass is routed to by its shape and format (csrc/gemm.hip, gemm_route): the K sum split
+over a workgroup's waves or over ranges, and the dense routes over operand-ordered and row-major weights, on every tile.
 
 Each shape: fp16 and fp32 inputs of equal values give equal bits; every output is the fp16 rounding of the exact
-(float64) sum of the fp16 operands up to ½ fp16 ulp + 2^-16·Σ|x·w| (an fp32 sum's rounding); an output with a row
-stride that rules out wide stores gets the same values and leaves its other columns alone."""
+(float64) sum of the fp16 operands up to ½ fp16 ulp + 2^-16·Σ|x·w| (an fp32 sum's rounding), and bitwise the one-range
+result where K is not split; an output with a row stride that rules out wide stores gets the same values and leaves its
+other columns alone."""
 import numpy as np
 import pytest
 import torch
@@ -14,20 +15,25 @@ from tests.test_gpu_prefill import check_f16_rounding
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
-# (rows, OUT, IN, groups): one shape or more per tile, with partial row blocks, one row, a single K step per wave,
-# uneven steps per wave, more steps than one block of scale words
-SHAPES = [
-    (1, 256, 256, 1), (17, 128, 512, 1), (16, 768, 5376, 1),          # 16 × 16
-    (33, 3072, 768, 1), (31, 1536, 2304, 3),                          # 32 × 16
-    (65, 2048, 1536, 1), (150, 1536, 512, 3),                         # 32 × 32
-    (130, 1024, 4096, 1),                                             # 64 × 16
-    (129, 2304, 768, 1), (90, 4096, 2304, 1),                         # 64 × 32
-    (257, 2304, 512, 1), (700, 768, 1024, 1),                         # 64 × 64
-    (1300, 512, 2048, 1),                                             # dense 64 × 64
-    (700, 2304, 768, 3), (1030, 1024, 1280, 1),                       # dense 64 × 128
-    (1001, 3072, 1024, 3), (1500, 2304, 256, 1),                      # dense 128 × 128
-    (1999, 4608, 512, 1),                                             # dense 256 × 256
-]
+# kernel and tile: (rows, OUT, IN, groups) with that route in all five formats (None: it differs between them); partial
+# row blocks, one row, a single K step per wave, uneven steps per wave, more steps than one block of scale words
+SHAPES = {
+    ("waves", 16, 16): [(1, 256, 256, 1), (17, 128, 512, 1), (16, 768, 5376, 1), (31, 1536, 2304, 3)],
+    ("waves", 32, 16): [(17, 2304, 256, 3), (257, 384, 768, 1), (128, 768, 768, 1), (96, 768, 3072, 1), (150, 1536, 512, 3),
+                        (128, 1024, 5376, 1)],
+    ("waves", 32, 32): [(31, 4608, 2048, 1), (129, 3072, 1024, 3), (129, 6144, 512, 1), (150, 3072, 5376, 1)],
+    ("waves", 64, 16): [(33, 3072, 768, 1), (65, 2048, 1536, 1), (190, 3840, 5376, 3)],
+    ("waves", 64, 32): [(257, 3840, 256, 3), (130, 2304, 2304, 1), (90, 4096, 2304, 1), (640, 640, 2304, 1)],
+    ("waves", 64, 64): [(65, 8192, 512, 1), (129, 4608, 512, 3), (900, 1024, 512, 1), (127, 8192, 1792, 1)],
+    ("dense", 64, 64): [(1030, 512, 2304, 1), (1100, 640, 3072, 1)],
+    ("dense", 64, 128): [(700, 2304, 768, 3), (1030, 1024, 1280, 1), (3001, 640, 1536, 1)],
+    ("dense", 128, 128): [(1001, 3072, 1024, 3), (257, 8192, 512, 1), (1300, 1920, 2048, 1)],
+    ("dense", 256, 256): [(1999, 4608, 2816, 3), (4100, 2048, 2816, 1)],
+    ("dense rows", 256, 256): [(1999, 4608, 512, 1), (1300, 6144, 256, 3)],
+    ("ranges", 128, 128): [(400, 8192, 256, 1), (1001, 3840, 256, 3)],
+    None: [(130, 1024, 4096, 1), (129, 2304, 768, 1), (257, 2304, 512, 1), (700, 768, 1024, 1), (1300, 512, 2048, 1),
+           (1500, 2304, 256, 1)],
+}
 
 
 def matrix(fmt, OUT, IN, seed):
@@ -51,19 +57,24 @@ def matrix(fmt, OUT, IN, seed):
 
 
 @pytest.mark.parametrize("fmt", ["sb6:0", "sb6:1", "sb6:2", "sym:8", "sym:6"])
-@pytest.mark.parametrize("M,OUT,IN,G", SHAPES)
-def test_quant_gemm_routes(fmt, M, OUT, IN, G):
-    print(f"[case] gemm route {fmt} M={M} {OUT}x{IN} G={G}", flush=True)
+@pytest.mark.parametrize("kernel,M,OUT,IN,G", [(k, *s) for k, v in SHAPES.items() for s in v])
+def test_quant_gemm_routes(fmt, kernel, M, OUT, IN, G):
+    print(f"[case] gemm route {kernel} {fmt} M={M} {OUT}x{IN} G={G}", flush=True)
     bufs, gemm, entry, bits, w16 = matrix(fmt, OUT, IN, M + OUT)
     per = OUT // G
+    route = Q.rwkvq_gemm_route(fmt[:3], bits, M, OUT, IN, per)
+    assert kernel in (None, route[:3])
     gen = torch.Generator(device=DEV).manual_seed(M + IN)
     x = torch.randn((G, M, IN), generator=gen, device=DEV).half()
+    dequants = f"{fmt[:3]}_dequant"
+    n0 = _lib.counters()[dequants]
     y = gemm(x, *bufs, OUT, IN, bits, out_per=per)
+    assert _lib.counters()[dequants] == n0 + route[0].startswith("dense")   # the kernel that the route names ran
     assert torch.equal(gemm(x.float(), *bufs, OUT, IN, bits, out_per=per), y)
-    rows = slice(0, M) if M < 300 else torch.tensor([*range(40), *range(M - 40, M)], device=DEV)
+    if route[3] == 1:
+        assert torch.equal(gemm(x, *bufs, OUT, IN, bits, out_per=per, split=False), y)
     for g in range(G):
-        xs, ws = x[g][rows].double(), w16[g * per:(g + 1) * per].double()
-        got = y[rows][:, g * per:(g + 1) * per]
+        xs, ws, got = x[g].double(), w16[g * per:(g + 1) * per].double(), y[:, g * per:(g + 1) * per]
         check_f16_rounding(got.cpu().numpy(), (xs @ ws.T).cpu().numpy(), (xs.abs() @ ws.abs().T).cpu().numpy())
     h = gemm(x, *bufs, OUT, IN, bits, out_per=per, epilogue="relu2_f16")
     assert torch.equal(h, (torch.relu(y) * torch.relu(y)).half())

@@ -146,8 +146,9 @@ def test_quant_gemm_layouts_epilogues_and_groups(orc, fmt, split):
 
 def test_quant_gemm_split_workspace_contract(orc):
     """The split long pass through the C-ABI: a workspace smaller than
-    rwkv_quant_gemm_workspace is refused (nothing launched, y untouched), a
-    NULL one runs as one K range, an adequate one gives the split sums."""
+    rwkv_quant_gemm_workspace is refused where K ranges would need as much
+    (nothing launched, y untouched), a NULL one runs as one K range, an
+    adequate one gives the split sums."""
     case("quant gemm workspace contract")
     from swiftrwkv_amd import _lib
     M, OUT, IN = 96, 768, 3072
@@ -175,12 +176,11 @@ def test_quant_gemm_split_workspace_contract(orc):
 
 @pytest.mark.parametrize("fmt", ["sb6:0", "sb6:2", "sym:8", "sym:6"])
 def test_quant_gemm_dense_route_bitwise(orc, fmt):
-    """Shapes with at least 128 output tiles of 256 × 256 and fp16 inputs:
-    given a workspace, the quantised entry points dequantise the weight into
-    it and run the dense fp16 kernel — bitwise the one-range fused launch
-    (the same products in the same order) for a fused group of three
-    matrices with a partial last row block, for every epilogue; and within
-    the fp16-base oracle's bound on a sample of rows."""
+    """A large pass: given a workspace, the quantised entry points dequantise
+    the weight into it and run a dense fp16 kernel — bitwise the one-range
+    fused launch (the same products in the same order) for a fused group of
+    three matrices with a partial last row block, for every epilogue; and
+    within the fp16-base oracle's bound on a sample of rows."""
     case(f"quant gemm dense route {fmt}")
     from swiftrwkv_amd import _lib
     M, D, IN = 2000, 1536, 512   # 8 row blocks × 18 feature blocks

@@ -740,13 +740,14 @@ def bench_prefill(dev, seconds_cap=60.0):
             return None
         x = torch.randn((M, IN), device=dev).to(torch.float16)
         fl = 2 * M * OUT * IN
-        # the long pass as the prefill calls it (with a workspace: the dequant
-        # plus the dense kernel where the shape takes that route)
+        # the long pass as the prefill calls it, by the kernel its shape takes
         ms = timed(lambda: Q.rwkvq_sb6_gemm(x, q[0], q[1], q[2], OUT, IN), 10) * 1e3
         tf = fl / (ms * 1e-3) / 1e12
         line = {"shape": f"{M}x{OUT}x{IN}", "ms": ms, "TFLOPs": tf, "mfma_fp16_peak_frac": tf / 2500.0,
-                "route": "dequant + dense" if Q.rwkvq_gemm_workspace(M, OUT, IN) == OUT * IN * 2 else "fused"}
-        # the fused kernel alone (no workspace) and the dense kernel alone
+                "route": "{} {}x{} /{}".format(*Q.rwkvq_gemm_route("sb6", 0, M, OUT, IN))}
+        # one K range on 128 x 128 tiles (quant_gemm_kernel), and the row-major
+        # dense kernel on a dense fp16 weight (dense_gemm_kernel: rwkv_f16_gemm's,
+        # not the operand-ordered dense_tiles_kernel that a large pass takes)
         ms_f = timed(lambda: Q.rwkvq_sb6_gemm(x, q[0], q[1], q[2], OUT, IN, split=False), 10) * 1e3
         line["fused_ms"], line["fused_peak_frac"] = ms_f, fl / (ms_f * 1e-3) / 1e12 / 2500.0
         if Q.rwkvq_f16_gemm_applies(M, OUT, IN):

@@ -120,8 +120,8 @@ rwkv_status rwkv_wkv7_train_fwd(const void* r, const void* w, const void* k, con
  * h_ckpt, sa: the training forward's outputs.  d_out [B,T,H,64] fp32;
  * d_h_out [B,H,64,64] fp32 or NULL.  Gradients dr..db [B,T,H,64] are written
  * in g_dt (the primal's dtype, :440,462); dh_in [B,H,64,64] fp32.
- * variant: 2 = the default (wkv7BackwardV2 = true; column-owned, states
- * recomputed forward from h_in / the previous checkpoint), 1 = the
+ * variant: 2 = the default (wkv7BackwardV2 = true; states recomputed
+ * forward from h_in / the previous checkpoint), 1 = the
  * reference's row-owned ckptBwdKernel (WKV7Train.swift:99-205: one wave per
  * head, states recovered by dividing by w, so the gradients formed from them,
  * dr / dw / da, carry the forward's rounding amplified by up to Π 1/w over a
@@ -309,9 +309,9 @@ rwkv_status rwkv_sym_gemv_ep(const float* x, int64_t N,
  * pass of X070Backbone.baseMatmul with an fp16 base (Sources/RWKVGen/X070Backbone.swift:337-356,
  * 733-739): y = fp16(fp16(x)·fp16(W)ᵀ) where fp16(W) is exactly the dequant
  * rwkv_sb6_dequant(out_dt = f16) stores, products summed in fp32, the sum
- * rounded to fp16 (the fp16 matmul's output) — computed from the K3 bytes
- * without writing the dense weight.  sb6 with 4, 5 or 6-bit codes (xbits
- * 0..2); OUT and out_per multiples of 128, IN of 256 (rwkv_sb6_gemm_applies).
+ * rounded to fp16 (the fp16 matmul's output) — computed from the K3 bytes,
+ * or from an fp16 copy of the weight in the caller's workspace.  sb6 with 4, 5
+ * or 6-bit codes (xbits 0..2); OUT and out_per multiples of 128, IN of 256 (rwkv_sb6_gemm_applies).
  * x [groups][M][lda] in x_dt (f32 or f16; groups = OUT / out_per, matrix g
  * at x + g·x_group_stride elements): output feature o reads group o / out_per,
  * so r/k/v with their own inputs run as one launch.  y [M][ldy]:
@@ -378,7 +378,8 @@ rwkv_status rwkv_sym_gemm_auto(const void* x, rwkv_dtype x_dt, int64_t M, int64_
  * epilogues.  256 × 256 output tiles: OUT and out_per multiples of 256, IN of
  * 128, lda >= IN and a multiple of 8, x and w 16-byte aligned
  * (rwkv_f16_gemm_applies for lda = IN).  Each output is rwkv_sb6_gemm's /
- * rwkv_sym_gemm's bitwise when w is the fp16 weight those decode. */
+ * rwkv_sym_gemm's bitwise when w is the fp16 weight those decode and they do
+ * not split K (NULL workspace). */
 int rwkv_f16_gemm_applies(int64_t M, int64_t OUT, int64_t IN, int64_t out_per);
 rwkv_status rwkv_f16_gemm(const void* x, int64_t M, int64_t lda, int64_t x_group_stride, const void* w, void* y,
                           int64_t ldy, int64_t OUT, int64_t IN, int64_t out_per, int epilogue, void* stream);

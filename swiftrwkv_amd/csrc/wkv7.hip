@@ -380,9 +380,9 @@ constexpr int NOUT = 6;   // dr dw dk db dv da
 // A chunk's 17 states are in registers (136 of 234), computed once: two windows
 // of eight steps repeat half of them.
 //
-// What bounds it: with 256 heads, one per CU, the issue of both waves of a SIMD
-// (the loads' and the barrier's latencies are hidden: loading the next step's
-// vectors early changes nothing).  8 × 4096 × 32 heads, bf16: 3.9 ms with the
+// What bounds it: with 256 heads, one per CU, mostly the issue of both waves of
+// a SIMD (0.35 of its cycles matrix, 0.29 vector instructions; loading the next
+// step's vectors early changes nothing), then the step's exchange through LDS.  8 × 4096 × 32 heads, bf16: 3.9 ms with the
 // vector ALU alone, whose products all take a broadcast operand, 3.0 ms so.  Four waves
 // of 16 rows (one per SIMD, half the LDS traffic): 4.7 ms.
 using f32x4 = __attribute__((ext_vector_type(4))) float;

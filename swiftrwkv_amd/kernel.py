@@ -195,8 +195,8 @@ def _train_forward(ins, dt, h0):
 
 
 class _WKV7Train(torch.autograd.Function):
-    """Forward: checkpointing kernel.  Backward: checkpoint kernel v2, column-owned
-    with recomputed states (or v1, the row-owned kernel that recovers them by
+    """Forward: checkpointing kernel.  Backward: checkpoint kernel v2, with
+    recomputed states (or v1, the row-owned kernel that recovers them by
     dividing by w, WKV7Train.swift:99-205), the VJP of wkv7TrainWithState
     (WKV7Train.swift:410-467).  Gradients come
     back in each primal's dtype; the state gradient in the state's dtype."""

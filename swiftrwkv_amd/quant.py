@@ -657,7 +657,8 @@ def rwkvq_f16_gemm(x, w, out_per: Optional[int] = None, epilogue: str = "store",
     (X070Backbone.swift:337-356 after the dequant): y [M, OUT] =
     fp16(x·wᵀ) with fp32 sums, x [M, IN] or [G, M, IN] fp16 (G = OUT /
     out_per, matrix g reading x[g]); epilogues as rwkvq_sb6_gemm.  Bitwise
-    the quantised GEMMs' result when w is the fp16 weight they decode."""
+    the quantised GEMMs' one-range result (split=False) when w is the fp16
+    weight they decode."""
     OUT, IN = w.shape
     per = OUT if out_per is None else out_per
     G = OUT // per

@@ -3,7 +3,7 @@ in parts:
 
 * WKV-7 training forward + backward at B8 T4096 H32 with bf16 inputs and
   gradients (the 1.5B training shape, B·H = 256: the sixteen-rows-per-wave
-  forward and the column-owned backward over 256 checkpoint chunks).  Every
+  forward and the eight-wave backward over 256 checkpoint chunks).  Every
   (batch, head) pair is an independent recurrence, so four (b, h) slices
   compared with the fp64 oracle run on those slices alone are exact checks of
   the full launch; the whole tensors are checked by properties (finite,

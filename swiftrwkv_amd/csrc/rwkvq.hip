@@ -841,14 +841,14 @@ __global__ __launch_bounds__(1024) void gemv_ln_kernel(typename Sb6Fmt<0>::Ptr P
 }
 
 // Batches (N ≥ 2 inputs): NT inputs share one pass over the weights.  The
-// lane's units and their order, the per-unit arithmetic (F::prep / F::apply)
+// lane → (row, unit) assignment, the per-unit arithmetic (F::prep / F::apply)
 // and the group sums are those of gemv_kernel, so every output is bitwise
 // what a single-input launch gives.  A unit's codes are decoded once for all
 // NT inputs.  blockIdx.y selects the tile of NT inputs.  The inputs are
 // staged in LDS a chunk of CP passes (CP·G units) at a time, so any IN fits
 // and a workgroup reads each input element once; the next pass's weights are
 // in flight during the current one.
-template <class F, int NT>
+template <class F, int RL, int NT>
 __global__ __launch_bounds__(512) void gemv_batch_kernel(const float* __restrict__ x, int N, typename F::Ptr P,
                                                          float* __restrict__ y, int OUT, int IN, int out_per,
                                                          GemvGeom geo, int CP) {
@@ -863,8 +863,8 @@ __global__ __launch_bounds__(512) void gemv_batch_kernel(const float* __restrict
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int gi = lane >> geo.LG, g = lane & (geo.G - 1);
-    const int row = (blockIdx.x * geo.WPB + wave) * geo.R + gi;
-    const int xi = NK == 1 ? 0 : min(row, OUT - 1) / out_per;
+    const int row0 = (blockIdx.x * geo.WPB + wave) * geo.R * RL + gi * RL;
+    const int xi = NK == 1 ? 0 : min(row0, OUT - 1) / out_per;   // RL divides out_per
     float inv = 1.0f;
     if constexpr (std::is_same_v<F, Sb6Fmt<0>>) {
         inv = __uint_as_float(0x7F000000u - __float_as_uint(__builtin_amdgcn_cvt_pk_f32_fp8(1, false)[0]));
@@ -872,7 +872,7 @@ __global__ __launch_bounds__(512) void gemv_batch_kernel(const float* __restrict
     // staged input rows: input nn, matrix k at nn·NK + k, or only the
     // workgroup's own matrix kwg (one_k) at nn
     const int NKs = geo.one_k ? 1 : NK;
-    const int kwg = geo.one_k ? (int)(blockIdx.x * geo.WPB * geo.R) / out_per : 0;
+    const int kwg = geo.one_k ? (int)(blockIdx.x * geo.WPB * geo.R * RL) / out_per : 0;
     const int rows = NT * NKs;
     const int CU = CP * geo.G;     // units per chunk
     const int XS = CU * 36;        // floats per staged row: units padded to 36 floats
@@ -880,8 +880,10 @@ __global__ __launch_bounds__(512) void gemv_batch_kernel(const float* __restrict
 
     using Raw = typename F::Raw;
     using Prep = typename F::Prep;
-    auto load_pass = [&](int p, Raw& W) __attribute__((always_inline)) {
-        F::load(P, NU, (uint32_t)min(row, OUT - 1), (uint32_t)(p * geo.G + g), W);
+    auto load_pass = [&](int p, Raw (&W)[RL]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rr = 0; rr < RL; ++rr)
+            F::load(P, NU, (uint32_t)min(row0 + rr, OUT - 1), (uint32_t)(p * geo.G + g), W[rr]);
     };
     auto stage = [&](int u0, int nu) __attribute__((always_inline)) {   // units u0 .. u0 + nu - 1
         const int q4 = nu * 8;   // float4 per staged row
@@ -923,10 +925,12 @@ __global__ __launch_bounds__(512) void gemv_batch_kernel(const float* __restrict
         }
     };
 
-    float acc[NT];
+    float acc[NT][RL];
 #pragma unroll
-    for (int nn = 0; nn < NT; ++nn) acc[nn] = 0.0f;
-    Raw W;
+    for (int nn = 0; nn < NT; ++nn)
+#pragma unroll
+        for (int rr = 0; rr < RL; ++rr) acc[nn][rr] = 0.0f;
+    Raw W[RL];
     load_pass(0, W);   // in flight while the first chunk is staged
     int u0 = 0;
 #pragma unroll 1
@@ -936,10 +940,11 @@ __global__ __launch_bounds__(512) void gemv_batch_kernel(const float* __restrict
             u0 = p * geo.G;
             stage(u0, min(CP, geo.NP - p) * geo.G);
         }
-        Raw Wn;
+        Raw Wn[RL];
         if (p + 1 < geo.NP) load_pass(p + 1, Wn);
-        Prep q;
-        F::prep(W, inv, q);
+        Prep q[RL];
+#pragma unroll
+        for (int rr = 0; rr < RL; ++rr) F::prep(W[rr], inv, q[rr]);
         const int lu = p * geo.G + g - u0;
         // inputs nn + 1 are read from LDS while input nn is applied; the fence
         // (it consumes the accumulators and orders memory) keeps at most two
@@ -964,16 +969,25 @@ __global__ __launch_bounds__(512) void gemv_batch_kernel(const float* __restrict
 #pragma unroll
         for (int nn = 0; nn < NT; ++nn) {
             if (nn + 1 < NT) read_x(nn + 1, xv[(nn + 1) & 1], xs[(nn + 1) & 1]);
-            acc[nn] = F::apply(q, xv[nn & 1], xs[nn & 1], acc[nn]);
-            asm volatile("" : "+v"(acc[nn]) : : "memory");
+#pragma unroll
+            for (int rr = 0; rr < RL; ++rr) {
+                acc[nn][rr] = F::apply(q[rr], xv[nn & 1], xs[nn & 1], acc[nn][rr]);
+                asm volatile("" : "+v"(acc[nn][rr]) : : "memory");
+            }
         }
-        if (p + 1 < geo.NP) W = Wn;
+        if (p + 1 < geo.NP) {
+#pragma unroll
+            for (int rr = 0; rr < RL; ++rr) W[rr] = Wn[rr];
+        }
     }
 #pragma unroll
-    for (int nn = 0; nn < NT; ++nn) {
-        const float t = group_sum(acc[nn], geo.G);
-        if (g == 0 && row < OUT && nn < N) store_out(y, (int64_t)nn * OUT + row, t, geo.ep);
-    }
+    for (int nn = 0; nn < NT; ++nn)
+#pragma unroll
+        for (int rr = 0; rr < RL; ++rr) {
+            const float t = group_sum(acc[nn][rr], geo.G);
+            const int row = row0 + rr;
+            if (g == 0 && row < OUT && nn < N) store_out(y, (int64_t)nn * OUT + row, t, geo.ep);
+        }
 }
 
 // ─────────────────────────────── host side ───────────────────────────────
@@ -1125,7 +1139,7 @@ constexpr int64_t kBatchLds = 160 * 1024;   // LDS of one gfx950 workgroup (and 
 
 struct BatchPlan {
     GemvGeom geo;
-    int NT, CP;
+    int RL, NT, CP;
     size_t lds;
     unsigned blocks;
 };
@@ -1147,16 +1161,22 @@ struct BatchPlan {
 // 156 registers instead of 101 and halve the waves in flight (sym_6 4096 × 1024
 // at N = 8: 7.7 against 6.7 µs, 14336 × 4096 at N = 16: 80 against 66; sym_8
 // 8192 × 2048 at N = 8: 11.6 against 11.1; sb6_4 2048 × 2048: 7.2 against 6.2;
-// no shape the other way by more than 1 %; four rows spill).  WPB = 8 waves
-// where the grid stays ≥ 256 workgroups, else 4.  CP passes per chunk fill the
-// LDS share.
+// four rows spill).  Where a row takes the whole wave (G = 64: IN of 6144 or
+// more, multiples of 2048) a workgroup of 8 waves has only 8 rows to show for
+// staging the inputs, and two per lane win where their workgroups, one per CU,
+// fill it: whole rounds of 256, or a last one more than half full (sb6_4 N = 16
+// 2048 × 14336: 37 against 41 µs, 4096 × 14336 72 against 78).  With fewer the
+// one-row kernel's workgroups, two per CU, take half a round less (3072 × 8192
+// at N = 16: 1.5 rounds, 44 against 38 µs; 900 points, 8192 and 14336 columns,
+// all on this line's side or within 4 % of a tie).  WPB = 8 waves where the
+// grid stays ≥ 256 workgroups, else 4.  CP passes per chunk fill the LDS share.
 bool plan_batch(int64_t OUT, int64_t NU, int64_t rl_div, int64_t N, int64_t NK, bool sums, BatchPlan& bp) {
     const GemvPlan one = plan_gemv(OUT, NU, rl_div, 1, NK, sums, false);
     bp.geo = one.geo;
     bp.geo.NP = (int)(NU / bp.geo.G);
     const int64_t per_row_pass = (int64_t)bp.geo.G * (36 + (sums ? 2 : 0)) * 4;   // bytes per input row, one pass
-    auto blocks = [&](int wpb) {
-        const int64_t per = (int64_t)wpb * bp.geo.R;
+    auto blocks = [&](int wpb, int rl) {
+        const int64_t per = (int64_t)wpb * bp.geo.R * rl;
         return (OUT + per - 1) / per;
     };
     auto tiles = [&](int nt) { return (N + nt - 1) / nt; };
@@ -1166,15 +1186,17 @@ bool plan_batch(int64_t OUT, int64_t NU, int64_t rl_div, int64_t N, int64_t NK, 
     bp.geo.one_k = NK > 1 && rl_div % (8 * (int64_t)bp.geo.R) == 0;
     const int64_t NKs = bp.geo.one_k ? 1 : NK;
     bp.NT = N > 4 ? 8 : 4;
-    if (bp.NT > 4 && (bp.NT * NKs * per_row_pass > kBatchLds / 2 || blocks(4) * tiles(bp.NT) < 1024)) bp.NT = 4;
-    if (bp.NT == 4 && (N <= 2 || (N <= 8 && blocks(4) * tiles(4) < 1024))) bp.NT = 2;
+    if (bp.NT > 4 && (bp.NT * NKs * per_row_pass > kBatchLds / 2 || blocks(4, 1) * tiles(bp.NT) < 1024)) bp.NT = 4;
+    if (bp.NT == 4 && (N <= 2 || (N <= 8 && blocks(4, 1) * tiles(4) < 1024))) bp.NT = 2;
     const int64_t pass_bytes = bp.NT * NKs * per_row_pass;
     if (pass_bytes > kBatchLds) return false;
     const int64_t budget = pass_bytes <= kBatchLds / 2 ? kBatchLds / 2 : kBatchLds;
     bp.CP = (int)std::min<int64_t>(bp.geo.NP, budget / pass_bytes);
     bp.lds = (size_t)(pass_bytes * bp.CP);
-    bp.geo.WPB = blocks(8) * tiles(bp.NT) >= 256 ? 8 : 4;
-    bp.blocks = (unsigned)blocks(bp.geo.WPB);
+    const int64_t two = blocks(8, 2) * tiles(bp.NT), last = two % 256;
+    bp.RL = bp.geo.R == 1 && rl_div % (bp.geo.one_k ? 16 : 2) == 0 && two >= 256 && (last == 0 || last > 128) ? 2 : 1;
+    bp.geo.WPB = blocks(8, bp.RL) * tiles(bp.NT) >= 256 ? 8 : 4;
+    bp.blocks = (unsigned)blocks(bp.geo.WPB, bp.RL);
     return true;
 }
 
@@ -1182,12 +1204,18 @@ template <class F>
 bool launch_batch(const BatchPlan& bp, hipStream_t st, const float* x, int N, typename F::Ptr P, float* y, int OUT,
                   int IN, int out_per) {
     const dim3 grid(bp.blocks, (unsigned)((N + bp.NT - 1) / bp.NT)), block(64 * bp.geo.WPB);
-#define RWKV_GB(NTV)                                                                                    \
-    rwkv::launch_lds(gemv_batch_kernel<F, NTV>, grid, block, bp.lds, st, x, N, P, y, OUT, IN, out_per, \
+#define RWKV_GB(RLV, NTV)                                                                                    \
+    rwkv::launch_lds(gemv_batch_kernel<F, RLV, NTV>, grid, block, bp.lds, st, x, N, P, y, OUT, IN, out_per, \
                      bp.geo, bp.CP)
-    if (bp.NT == 8) RWKV_GB(8);
-    else if (bp.NT == 4) RWKV_GB(4);
-    else RWKV_GB(2);
+    if (bp.RL == 2) {
+        if (bp.NT == 8) RWKV_GB(2, 8);
+        else if (bp.NT == 4) RWKV_GB(2, 4);
+        else RWKV_GB(2, 2);
+    } else {
+        if (bp.NT == 8) RWKV_GB(1, 8);
+        else if (bp.NT == 4) RWKV_GB(1, 4);
+        else RWKV_GB(1, 2);
+    }
 #undef RWKV_GB
     return true;
 }

@@ -266,6 +266,29 @@ def test_batched_fused_gemv_matrix_sizes_bitwise(orc, OUT, IN):
                 assert torch.equal(fused[n:n + 1, i * OUT:(i + 1) * OUT], alone), (i, n)
 
 
+# two rows per lane: rows that take a whole wave (6144 columns or more), from 256 workgroups on unless a last round of
+# them is up to half full: partial last rows, odd sizes, fused groups staging one matrix or all three
+@pytest.mark.parametrize("OUT,IN,Kn,N", [(510, 6144, 1, 32), (512, 6144, 1, 32), (509, 6144, 1, 32), (544, 6144, 1, 32),
+                                         (256, 6144, 3, 36), (252, 6144, 3, 36), (264, 8192, 3, 36), (768, 8192, 1, 31)])
+def test_batched_gemv_wide_rows_bitwise(orc, OUT, IN, Kn, N):
+    case(f"batched sym / sb6 {Kn}x{OUT}x{IN} N={N}")
+    x = np.random.default_rng(OUT + IN).standard_normal((N * Kn, IN)).astype(np.float32)
+    for make, run in ((lambda i: sb6_tensor(orc, OUT, IN, 0, seed=60 + i),
+                       lambda z, w, o, per: Q.rwkvq_sb6_gemv(z, *w, o, IN, 0, out_per=per)),
+                      (lambda i: sb6_tensor(orc, OUT, IN, 2, seed=60 + i),
+                       lambda z, w, o, per: Q.rwkvq_sb6_gemv(z, *w, o, IN, 2, out_per=per)),
+                      (lambda i: sym_tensor(orc, OUT, IN, 8, seed=60 + i),
+                       lambda z, w, o, per: Q.rwkvq_sym_gemv(z, *w, o, IN, 8, out_per=per))):
+        parts = [make(i) for i in range(Kn)]
+        w = [dev(np.concatenate([p[j] for p in parts])) for j in range(3)]
+        fused = run(dev(x), w, OUT * Kn, OUT if Kn > 1 else None)
+        for i, p in enumerate(parts):
+            wi = [dev(z) for z in p]
+            for n in range(N):
+                alone = run(dev(x[n * Kn + i:n * Kn + i + 1]), wi, OUT, None)
+                assert torch.equal(fused[n:n + 1, i * OUT:(i + 1) * OUT], alone), (i, n)
+
+
 def test_gemv_is_deterministic(orc):
     case("gemv determinism")
     qblk, qsqm, ddm = sb6_tensor(orc, 3072, 768, 1, seed=3)

@@ -479,7 +479,8 @@ __global__ __launch_bounds__(256) void gemm_split_reduce(const float* __restrict
 // one tile of 16·MT × 16·NT outputs and its W waves take K / W columns each.
 // A wave works alone: it moves 128 columns at a time (its input rows and its
 // weight rows' packed bytes) through its own LDS region, so no barrier stands
-// in the K loop, with the next 128 columns' loads in registers meanwhile; the
+// in the K loop (a wave's LDS operations run in order, so what it stages is
+// there for its own reads), with the next 128 columns' loads in registers meanwhile; the
 // W partial tiles meet in LDS at the end, summed in wave order
 // (deterministic), where the epilogue is applied.  One launch.
 //
